@@ -1,0 +1,65 @@
+"""The bit-parallel depth field (vrt_field.h) against the oracle's
+fixDepthField, word for word: sizes around the tile (32 x 8 x 16 voxels) and
+the bitmap's words, densities from one solid voxel to nearly full, and empty
+voxels that already hold other words.  The padded copy that the build writes
+is read back through rays."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def random_world(rng, dims, density):
+    n = dims[0] * dims[1] * dims[2]
+    w = np.full(n, -1, np.int32)
+    # empty voxels holding some jump already: nearer than 2 cells they keep it
+    old = rng.random(n) < 0.3
+    w[old] = (-np.sqrt(rng.integers(4, 37, int(old.sum())).astype(np.float32))).view(np.int32)
+    solid = rng.random(n) < density
+    solid[rng.integers(0, n)] = True
+    w[solid] = rng.integers(0, 1 << 24, int(solid.sum()))
+    return w
+
+
+def check_rays(gpu, orc, ctx, words, dims, rng, n=4000):
+    start = np.stack([rng.uniform(-1.5, d + 1.5, n) for d in dims], 1).astype(np.float32)
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    dist = rng.integers(1, 200, n).astype(np.int32)
+    g = ctx.cast_rays(start, d, dist, 256)
+    r = orc.cast_rays(words, dims, start, d, dist, 256)
+    for k in ("hit", "face", "steps"):
+        assert np.array_equal(g[k], r[k]), "%s differs for %d rays" % (k, int((g[k] != r[k]).sum()))
+
+
+DIMS = [(1, 1, 1), (31, 7, 15), (32, 8, 16), (33, 9, 17), (34, 8, 16), (63, 16, 33), (64, 15, 32), (65, 17, 31),
+        (66, 3, 50), (127, 25, 2), (130, 40, 47), (16, 30, 64), (5, 64, 5)]
+
+
+@pytest.mark.parametrize("dims", DIMS, ids=["%dx%dx%d" % d for d in DIMS])
+@pytest.mark.parametrize("density", [0.0, 0.002, 0.05, 0.97])
+def test_build_equals_oracle(gpu, orc, dims, density):
+    rng = np.random.default_rng(dims[0] * 7919 + dims[1] * 31 + dims[2] + int(density * 1000))
+    world = random_world(rng, dims, density)
+    ctx = gpu.Context(dims)
+    ctx.upload(world)
+    ctx.build_depth_field()
+    got, ref = ctx.download(), orc.depth_field(world, dims)
+    assert np.array_equal(got, ref), "%d voxels differ" % int((got != ref).sum())
+    check_rays(gpu, orc, ctx, ref, dims, rng)
+    ctx.close()
+
+
+def test_build_around_one_voxel_at_every_place_in_a_tile(gpu, orc):
+    """One solid voxel, at places that cover every x in a bitmap word and every
+    (y, z) of a tile: all distance classes, across every kind of tile border."""
+    dims = (96, 24, 48)
+    ctx = gpu.Context(dims)
+    for k in range(32):
+        x, y, z = 32 + k, 8 + k % 8, 16 + (k * 5) % 16
+        world = np.full(dims[0] * dims[1] * dims[2], -1, np.int32)
+        world[x + dims[0] * (y + dims[1] * z)] = 0x203040
+        ctx.upload(world)
+        ctx.build_depth_field()
+        got, ref = ctx.download(), orc.depth_field(world, dims)
+        assert np.array_equal(got, ref), "voxel (%d, %d, %d): %d differ" % (x, y, z, int((got != ref).sum()))
+    ctx.close()

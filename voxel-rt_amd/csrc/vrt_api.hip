@@ -253,6 +253,20 @@ int upload_table(vrt_ctx* c) {
     return VRT_OK;
 }
 
+// The distinct distances of the table in (-6, -2], largest first, as words.
+int make_field_words(vrt_ctx* c) {
+    std::vector<float> levels;
+    for (auto& e : reference_table())
+        if (e.dist > -6.0f && !(e.dist > -2.0f)) levels.push_back(e.dist);
+    std::sort(levels.begin(), levels.end(), [](float a, float b) { return a > b; });
+    levels.erase(std::unique(levels.begin(), levels.end()), levels.end());
+    if ((int)levels.size() != kFieldLevels) return fail(VRT_ERR_INVALID, "unexpected number of depth-field distances");
+    levels.push_back(-6.0f);
+    c->words.word[0] = 0;
+    std::memcpy(c->words.word + 1, levels.data(), levels.size() * sizeof(float));
+    return VRT_OK;
+}
+
 void release(vrt_ctx* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
@@ -266,7 +280,6 @@ void release(vrt_ctx* c) {
     if (c->table_dist) (void)hipFree(c->table_dist);
     if (c->table_rows) (void)hipFree(c->table_rows);
     if (c->table_rows_dist) (void)hipFree(c->table_rows_dist);
-    if (c->bricks) (void)hipFree(c->bricks);
     if (c->solid_bits) (void)hipFree(c->solid_bits);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
@@ -450,9 +463,8 @@ int vrt_create(vrt_ctx** out, int64_t X, int64_t Y, int64_t Z, int32_t device) {
         return bail(hip_fail(e, "hipMalloc counters"));
     if ((e = hipMalloc(&c->parts, (size_t)kPartsCap * sizeof(unsigned long long))) != hipSuccess)
         return bail(hip_fail(e, "hipMalloc partial counts"));
-    const uint64_t nbricks = (uint64_t)((X + 7) / 8) * ((Y + 7) / 8) * ((Z + 7) / 8);
-    if ((e = hipMalloc(&c->bricks, nbricks)) != hipSuccess) return bail(hip_fail(e, "hipMalloc bricks"));
     int rc = upload_table(c);
+    if (!rc) rc = make_field_words(c);
     if (rc) return bail(rc);
     if ((e = hipMemsetAsync(c->counters, 0, counter_bytes, c->stream)) != hipSuccess)
         return bail(hip_fail(e, "hipMemsetAsync"));
@@ -701,8 +713,7 @@ int vrt_build_depth_field(vrt_ctx* ctx) {
             return fail(VRT_ERR_NOMEM, "cannot allocate the depth-field build's solidity bitmap");
         }
     }
-    if (int rc = launch_build_depth_field(g, ctx->table, ctx->bricks, ctx->solid_bits, ctx->stream)) return rc;
-    return refresh_render_all(ctx);
+    return launch_build_depth_field(g, ctx->rgrid, ctx->words, ctx->solid_bits, ctx->stream);
 }
 
 // fixDepthField, src/render.cpp:226-253, over a box.

@@ -118,6 +118,14 @@ struct ViewDesc {
     int64_t first_tile;    // prefix sum of tiles over earlier views
 };
 
+// The words that a depth field can give an empty voxel, nearest first
+// (vrt_field.h): entry 0 is unused (the word is left as it was), entries 1 to
+// kFieldLevels the bits of the table's distances in (-6, -2], the last -6.0f.
+constexpr int kFieldLevels = 23;
+struct FieldWords {
+    int32_t word[kFieldLevels + 2];
+};
+
 struct DepthTableDev {
     const int32_t* packed;  // (dx+8) | (dy+8)<<5 | (dz+8)<<10, sorted by dist descending
     const float* dist;      // dist of each packed entry
@@ -162,9 +170,10 @@ int launch_fix_depth_box(const GridDesc& g, const DepthTableDev& t, int32_t x0, 
                          int32_t x1, int32_t y1, int32_t z1, int32_t sphere_cx, int32_t sphere_cy,
                          int32_t sphere_cz, int32_t sphere_r, hipStream_t s);
 // Whole-grid depth field: solidity bitmap (Y*Z rows of solid_bits_words(g)
-// words), brick flags (one byte per 8x8x8 brick), then the brick kernel.
+// words), then every tile's words into the grid and into `render`, the
+// padded copy of the whole grid.
 uint32_t solid_bits_words(const GridDesc& g);
-int launch_build_depth_field(const GridDesc& g, const DepthTableDev& t, uint8_t* bricks, uint32_t* bits,
+int launch_build_depth_field(const GridDesc& g, const GridDesc& render, const FieldWords& words, uint32_t* bits,
                              hipStream_t s);
 int launch_carve_sphere(const GridDesc& g, int32_t cx, int32_t cy, int32_t cz, int32_t r, hipStream_t s);
 int launch_set_voxel(const GridDesc& g, int64_t index, int32_t y, int32_t v, hipStream_t s);
@@ -217,7 +226,7 @@ struct vrt_ctx {
     int32_t* table_rows = nullptr;
     float* table_rows_dist = nullptr;
     vrt::DepthTableDev table{};
-    uint8_t* bricks = nullptr;
+    vrt::FieldWords words{};
     uint32_t* solid_bits = nullptr;  // whole-grid build scratch, allocated by the first build
     int32_t num_cus = 0;
     bool tuned = false;
