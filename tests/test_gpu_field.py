@@ -63,3 +63,49 @@ def test_build_around_one_voxel_at_every_place_in_a_tile(gpu, orc):
         got, ref = ctx.download(), orc.depth_field(world, dims)
         assert np.array_equal(got, ref), "voxel (%d, %d, %d): %d differ" % (x, y, z, int((got != ref).sum()))
     ctx.close()
+
+
+def build(gpu, orc, dims, density, seed):
+    rng = np.random.default_rng(seed)
+    world = random_world(rng, dims, density)
+    ctx = gpu.Context(dims)
+    ctx.upload(world)
+    ctx.build_depth_field()
+    return rng, ctx, orc.depth_field(world, dims)
+
+
+@pytest.mark.parametrize("radius", [-3, -2, -1, 0, 1, 2, 5, 8, 13, 14, 40])
+@pytest.mark.parametrize("density", [0.01, 0.6])
+def test_remove_sphere_equals_oracle(gpu, orc, radius, density):
+    """Carve, repair and render copy in one launch: boxes of one and several
+    tiles (32 x 8 x 8), clipped at corners and faces, overlapping, with centres
+    in and outside the grid."""
+    dims = (75, 41, 58)
+    rng, ctx, ref = build(gpu, orc, dims, density, 100 + radius)
+    centres = [(0, 0, 0), (dims[0] - 1, dims[1] - 1, dims[2] - 1), (37, 20, 29), (38, 21, 30), (-2, 20, 70),
+               (31, 8, 8)] + [tuple(int(rng.integers(0, d)) for d in dims) for _ in range(3)]
+    for c in centres:
+        orc.remove_sphere(ref, dims, c, radius)
+        ctx.remove_sphere(*c, radius)
+    got = ctx.download()
+    assert np.array_equal(got, ref), "%d voxels differ" % int((got != ref).sum())
+    check_rays(gpu, orc, ctx, ref, dims, rng)
+    ctx.close()
+
+
+@pytest.mark.parametrize("lo,hi", [((0, 0, 0), (75, 41, 58)), ((5, 3, 9), (6, 4, 10)), ((10, 7, 1), (43, 16, 9)),
+                                   ((-9, 30, 40), (200, 90, 99)), ((33, 1, 1), (33, 9, 9))])
+def test_fix_box_equals_oracle(gpu, orc, lo, hi):
+    dims = (75, 41, 58)
+    rng = np.random.default_rng(sum(lo) + sum(hi))
+    world = random_world(rng, dims, 0.03)
+    ctx = gpu.Context(dims)
+    ctx.upload(world)
+    ctx.fix_depth_field_box(lo, hi)
+    box = tuple(slice(max(0, lo[k]), max(0, min(dims[k], hi[k]))) for k in (2, 1, 0))
+    ref = world.copy()
+    ref.reshape(dims[::-1])[box] = orc.depth_field(world, dims).reshape(dims[::-1])[box]
+    got = ctx.download()
+    assert np.array_equal(got, ref), "%d voxels differ" % int((got != ref).sum())
+    check_rays(gpu, orc, ctx, ref, dims, rng)
+    ctx.close()

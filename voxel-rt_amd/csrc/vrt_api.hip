@@ -197,62 +197,6 @@ int check_ctx(vrt_ctx* c) {
     return VRT_OK;
 }
 
-// Depth table on the device, sorted by decreasing distance, entries at -6
-// (never counted: the test at src/render.cpp:240 is strict) dropped.
-int upload_table(vrt_ctx* c) {
-    auto t = reference_table();
-    std::vector<int> order(t.size());
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return t[a].dist > t[b].dist; });
-    std::vector<int32_t> packed;
-    std::vector<float> dist;
-    int32_t n_near = 0;
-    for (int i : order) {
-        if (!(t[i].dist > -6.0f)) continue;
-        packed.push_back((t[i].x + 8) | ((t[i].y + 8) << 5) | ((t[i].z + 8) << 10));
-        dist.push_back(t[i].dist);
-        if (t[i].dist > -2.0f) n_near++;
-    }
-    VRT_HIP(hipMalloc(&c->table_packed, packed.size() * sizeof(int32_t)));
-    VRT_HIP(hipMalloc(&c->table_dist, dist.size() * sizeof(float)));
-    VRT_HIP(hipMemcpy(c->table_packed, packed.data(), packed.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    VRT_HIP(hipMemcpy(c->table_dist, dist.data(), dist.size() * sizeof(float), hipMemcpyHostToDevice));
-    c->table.packed = c->table_packed;
-    c->table.dist = c->table_dist;
-    c->table.n = (int32_t)packed.size();
-    c->table.n_near = n_near;
-    // rows: the entries of one distance and one (dy, dz), their dx as a mask
-    std::vector<int32_t> rows;
-    std::vector<float> rows_dist;
-    int32_t n_rows_near = 0;
-    for (size_t a = 0; a < packed.size();) {
-        size_t e = a;
-        while (e < packed.size() && dist[e] == dist[a]) e++;  // one distance level
-        for (size_t i = a; i < e; i++) {
-            const int32_t dy = (packed[i] >> 5) & 31, dz = (packed[i] >> 10) & 31;
-            bool seen = false;
-            for (size_t j = a; j < i; j++) seen |= ((packed[j] >> 5) & 31) == dy && ((packed[j] >> 10) & 31) == dz;
-            if (seen) continue;
-            int32_t mask = 0;
-            for (size_t j = i; j < e; j++)
-                if (((packed[j] >> 5) & 31) == dy && ((packed[j] >> 10) & 31) == dz) mask |= 1 << ((packed[j] & 31) - 1);
-            rows.push_back(mask | (dy << 16) | (dz << 21));
-            rows_dist.push_back(dist[a]);
-            if (dist[a] > -2.0f) n_rows_near++;
-        }
-        a = e;
-    }
-    VRT_HIP(hipMalloc(&c->table_rows, rows.size() * sizeof(int32_t)));
-    VRT_HIP(hipMalloc(&c->table_rows_dist, rows_dist.size() * sizeof(float)));
-    VRT_HIP(hipMemcpy(c->table_rows, rows.data(), rows.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    VRT_HIP(hipMemcpy(c->table_rows_dist, rows_dist.data(), rows_dist.size() * sizeof(float), hipMemcpyHostToDevice));
-    c->table.rows = c->table_rows;
-    c->table.rows_dist = c->table_rows_dist;
-    c->table.n_rows = (int32_t)rows.size();
-    c->table.n_rows_near = n_rows_near;
-    return VRT_OK;
-}
-
 // The distinct distances of the table in (-6, -2], largest first, as words.
 int make_field_words(vrt_ctx* c) {
     std::vector<float> levels;
@@ -276,10 +220,6 @@ void release(vrt_ctx* c) {
     if (c->grid.top) (void)hipFree(c->grid.top);
     if (c->counters) (void)hipFree(c->counters);
     if (c->parts) (void)hipFree(c->parts);
-    if (c->table_packed) (void)hipFree(c->table_packed);
-    if (c->table_dist) (void)hipFree(c->table_dist);
-    if (c->table_rows) (void)hipFree(c->table_rows);
-    if (c->table_rows_dist) (void)hipFree(c->table_rows_dist);
     if (c->solid_bits) (void)hipFree(c->solid_bits);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
@@ -337,12 +277,7 @@ int solid_top_full(vrt_ctx* c) {
 }
 
 int refresh_render(vrt_ctx* c, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1) {
-    return refresh_render_on(c, c->stream, x0, y0, z0, x1, y1, z1);
-}
-
-int refresh_render_on(vrt_ctx* c, hipStream_t s, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1,
-                      int64_t z1) {
-    return refresh_copy_on(c, c->rgrid, s, x0, y0, z0, x1, y1, z1);
+    return refresh_copy_on(c, c->rgrid, c->stream, x0, y0, z0, x1, y1, z1);
 }
 
 int refresh_copy_on(vrt_ctx* c, const GridDesc& dst, hipStream_t s, int64_t x0, int64_t y0, int64_t z0, int64_t x1,
@@ -357,29 +292,26 @@ int refresh_copy_on(vrt_ctx* c, const GridDesc& dst, hipStream_t s, int64_t x0, 
     return launch_copy_box(c->grid, dst, x0, y0, z0, x1 - x0, y1 - y0, z1 - z0, s);
 }
 
-int remove_sphere_grid(vrt_ctx* c, int32_t cx, int32_t cy, int32_t cz, int32_t radius, hipStream_t s) {
-    if (int rc = launch_carve_sphere(c->grid, cx, cy, cz, radius, s)) return rc;
-    const int32_t R = radius + (VRT_DEPTH_FIELD_RADIUS >> 1);
-    if (R > 0) {
-        const int64_t x0 = (int64_t)cx - R, x1 = (int64_t)cx + R, y0 = (int64_t)cy - R, y1 = (int64_t)cy + R,
-                      z0 = (int64_t)cz - R, z1 = (int64_t)cz + R;
-        auto c32 = [](int64_t v) { return (int32_t)std::max<int64_t>(INT32_MIN, std::min<int64_t>(INT32_MAX, v)); };
-        if (int rc = launch_fix_depth_box(c->grid, c->table, c32(x0), c32(y0), c32(z0), c32(x1), c32(y1), c32(z1),
-                                          cx, cy, cz, R, s))
-            return rc;
-    }
-    return VRT_OK;
+namespace {
+// Half width of the box that a removeSphere can touch: the carve covers
+// [c - |r|, c + |r|) at most, the repair [c - R, c + R) with R = r + 3.
+int64_t sphere_reach(int32_t radius) {
+    const int64_t R = (int64_t)radius + (VRT_DEPTH_FIELD_RADIUS >> 1);
+    return std::max<int64_t>(radius < 0 ? -(int64_t)radius : (int64_t)radius, R);
 }
+}  // namespace
 
-int remove_sphere_refresh(vrt_ctx* c, int32_t cx, int32_t cy, int32_t cz, int32_t radius, hipStream_t s) {
-    return remove_sphere_refresh_into(c, c->rgrid, cx, cy, cz, radius, s);
+int remove_sphere_on(vrt_ctx* c, const GridDesc& render, int32_t cx, int32_t cy, int32_t cz, int32_t radius,
+                     hipStream_t s) {
+    const int32_t R = std::max(0, radius + (VRT_DEPTH_FIELD_RADIUS >> 1));
+    const int64_t M = sphere_reach(radius);
+    return launch_edit_box(c->grid, render, c->words, (int64_t)cx - M, (int64_t)cy - M, (int64_t)cz - M,
+                           (int64_t)cx + M, (int64_t)cy + M, (int64_t)cz + M, cx, cy, cz, R, radius, s);
 }
 
 int remove_sphere_refresh_into(vrt_ctx* c, const GridDesc& dst, int32_t cx, int32_t cy, int32_t cz, int32_t radius,
                                hipStream_t s) {
-    // the carve covers [c - |r|, c + |r|) at most, the repair [c - R, c + R)
-    const int64_t R = (int64_t)radius + (VRT_DEPTH_FIELD_RADIUS >> 1);
-    const int64_t M = std::max<int64_t>(radius < 0 ? -(int64_t)radius : (int64_t)radius, R);
+    const int64_t M = sphere_reach(radius);
     return refresh_copy_on(c, dst, s, (int64_t)cx - M, (int64_t)cy - M, (int64_t)cz - M, (int64_t)cx + M,
                            (int64_t)cy + M, (int64_t)cz + M);
 }
@@ -463,8 +395,7 @@ int vrt_create(vrt_ctx** out, int64_t X, int64_t Y, int64_t Z, int32_t device) {
         return bail(hip_fail(e, "hipMalloc counters"));
     if ((e = hipMalloc(&c->parts, (size_t)kPartsCap * sizeof(unsigned long long))) != hipSuccess)
         return bail(hip_fail(e, "hipMalloc partial counts"));
-    int rc = upload_table(c);
-    if (!rc) rc = make_field_words(c);
+    int rc = make_field_words(c);
     if (rc) return bail(rc);
     if ((e = hipMemsetAsync(c->counters, 0, counter_bytes, c->stream)) != hipSuccess)
         return bail(hip_fail(e, "hipMemsetAsync"));
@@ -719,17 +650,14 @@ int vrt_build_depth_field(vrt_ctx* ctx) {
 // fixDepthField, src/render.cpp:226-253, over a box.
 int vrt_fix_depth_field_box(vrt_ctx* ctx, int32_t x0, int32_t y0, int32_t z0, int32_t x1, int32_t y1, int32_t z1) {
     if (int rc = check_ctx(ctx)) return rc;
-    if (int rc = launch_fix_depth_box(ctx->grid, ctx->table, x0, y0, z0, x1, y1, z1, 0, 0, 0, -1, ctx->stream))
-        return rc;
-    return refresh_render(ctx, x0, y0, z0, x1, y1, z1);
+    return launch_edit_box(ctx->grid, ctx->rgrid, ctx->words, x0, y0, z0, x1, y1, z1, 0, 0, 0, -1, 0, ctx->stream);
 }
 
 // removeSphere, src/level.cpp:30-56.
 int vrt_remove_sphere(vrt_ctx* ctx, int32_t cx, int32_t cy, int32_t cz, int32_t radius) {
     if (int rc = check_ctx(ctx)) return rc;
     if (radius < -3 || radius > 4096) return fail(VRT_ERR_INVALID, "radius must be in [-3, 4096]");
-    if (int rc = remove_sphere_grid(ctx, cx, cy, cz, radius, ctx->stream)) return rc;
-    return remove_sphere_refresh(ctx, cx, cy, cz, radius, ctx->stream);
+    return remove_sphere_on(ctx, ctx->rgrid, cx, cy, cz, radius, ctx->stream);
 }
 
 // placeVoxel, src/render.cpp:256-262.
@@ -737,10 +665,9 @@ int vrt_place_voxel(vrt_ctx* ctx, int32_t x, int32_t y, int32_t z, int32_t voxel
     if (int rc = check_ctx(ctx)) return rc;
     const GridDesc& g = ctx->grid;
     if (x < 0 || y < 0 || z < 0 || (uint32_t)x >= g.X || (uint32_t)y >= g.Y || (uint32_t)z >= g.Z) return VRT_OK;
-    if (int rc = launch_set_voxel(g, (int64_t)x + (int64_t)g.X * y + (int64_t)g.XY * z, y, voxel, ctx->stream))
-        return rc;
+    if (int rc = launch_set_voxel(g, ctx->rgrid, x, y, z, voxel, ctx->stream)) return rc;
     if (voxel >= 0) ctx->top_host = std::max(ctx->top_host, y);  // as k_set_voxel raises *top
-    return refresh_render(ctx, x, y, z, (int64_t)x + 1, (int64_t)y + 1, (int64_t)z + 1);
+    return VRT_OK;
 }
 
 // destroyVoxel, src/render.cpp:265-271.

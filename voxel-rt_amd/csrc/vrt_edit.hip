@@ -7,9 +7,7 @@
 // The result depends only on which neighbours are solid, and a jump word is
 // negative (never solid), so every voxel of a region can be fixed in
 // parallel, in place, with the same result as the reference's sequential
-// loops.  Whole-grid builds compute d* on bit masks, 32 voxels at a time
-// (vrt_field.h); boxes scan the table in order of decreasing distance, so the
-// first solid neighbour found is d*.
+// loops.  d* is computed on bit masks, 32 voxels at a time (vrt_field.h).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,8 +18,6 @@
 namespace vrt {
 
 namespace {
-
-constexpr int32_t kMinus6Bits = (int32_t)0xC0C00000;  // bits of -6.0f
 
 // Solidity bitmap of the grid: row (y, z) is W words, bit x + 16 of the row is
 // voxel x (bits of x < 0 and x >= X are 0), so the 64 voxels from 16 before x0
@@ -64,63 +60,6 @@ __global__ void __launch_bounds__(256) k_solid_bits(GridDesc g, uint32_t* __rest
         w |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x141, 0xf, 0xf, true);  // the other four of eight
         if ((threadIdx.x & 7) == 0 && r0 + j < rows) bits[(r0 + j) * W + (q >> 3)] = w;
     }
-}
-
-constexpr int32_t kHalo = 7;
-constexpr int32_t kSpan = 8 + 2 * kHalo;  // 22 cells per row of the neighbourhood
-
-// fixDepthField's result for the voxel at (lx, ly, lz) of a brick whose
-// 22x22x22 neighbourhood solidity is in `rows` (bit b of row (ry, rz) is
-// x = lx - 7 + b).  The table is grouped by (distance, dy, dz): the first
-// group with a solid neighbour gives d*, as the first solid entry of the
-// sorted table would, and the group's dx mask (bit dx + 7) lines up with the
-// row shifted right by lx.  Eight groups per step keep eight LDS reads in
-// flight.
-__device__ __forceinline__ int32_t scan_groups(const uint32_t* rows, const DepthTableDev& t, int32_t lx, int32_t ly,
-                                               int32_t lz, int32_t old) {
-    const int32_t my_row = (lz + kHalo) * kSpan + ly + kHalo;
-    auto hits = [&](int32_t r) {
-        const int32_t dy = ((r >> 16) & 31) - 8, dz = ((r >> 21) & 31) - 8;
-        return ((rows[my_row + dz * kSpan + dy] >> lx) & (uint32_t)(r & 0x7fff)) != 0u;
-    };
-    int32_t found = -1;
-    int32_t k = 0;
-    for (; k + 8 <= t.n_rows; k += 8) {
-        uint32_t m = 0;
-#pragma unroll
-        for (int j = 0; j < 8; j++) m |= (uint32_t)hits(t.rows[k + j]) << j;
-        if (m) {
-            found = k + __builtin_ctz(m);
-            break;
-        }
-    }
-    if (found < 0)
-        for (; k < t.n_rows; k++)
-            if (hits(t.rows[k])) {
-                found = k;
-                break;
-            }
-    if (found < 0) return kMinus6Bits;
-    return found < t.n_rows_near ? old : __float_as_int(t.rows_dist[found]);
-}
-
-// The neighbourhood solidity of the brick at (bx0, by0, bz0) read from the
-// grid itself: thread r < 484 gathers the 22 voxels of row r (independent
-// loads, all in flight) into one word.
-__device__ __forceinline__ void fill_rows_from_grid(const GridDesc& g, uint32_t* rows, int32_t bx0, int32_t by0,
-                                                    int32_t bz0, int32_t c) {
-    if (c >= kSpan * kSpan) return;
-    const int32_t gy = by0 - kHalo + c % kSpan, gz = bz0 - kHalo + c / kSpan;
-    uint32_t v = 0;
-    if (((uint32_t)gy < g.Y) & ((uint32_t)gz < g.Z)) {
-        const int32_t* row = g.vox + (uint64_t)g.X * (uint64_t)gy + g.XY * (uint64_t)gz;
-#pragma unroll
-        for (int32_t b = 0; b < kSpan; b++) {
-            const int32_t gx = bx0 - kHalo + b;
-            if ((uint32_t)gx < g.X && row[gx] >= 0) v |= 1u << b;
-        }
-    }
-    rows[c] = v;
 }
 
 // Whole-grid build: one workgroup per tile of 32 x 8 x 16 voxels, whose
@@ -224,52 +163,107 @@ __global__ void __launch_bounds__(kTileThreads) k_field_tiles(GridDesc g, GridDe
     }
 }
 
-// fixDepthField over the box [x0,x1) x [y0,y1) x [z0,z1) (already clipped);
-// with sr >= 0 only voxels with (x-cx)^2+(y-cy)^2+(z-cz)^2 < sr^2.  The box
-// is tiled into 8x8x8 bricks from its corner, one workgroup each: the
-// brick's neighbourhood solidity is gathered from the grid into LDS and its
-// voxels scan the grouped table against it.
-__global__ void __launch_bounds__(512) k_fix_depth_box(GridDesc g, DepthTableDev t, int32_t x0, int32_t y0,
-                                                        int32_t z0, int32_t w, int32_t h, int32_t d, int32_t nbx,
-                                                        int32_t nby, int32_t cx, int32_t cy, int32_t cz, int32_t sr) {
-    __shared__ uint32_t rows[kSpan * kSpan];
-    const int32_t b = (int32_t)blockIdx.x;
-    const int32_t bx0 = x0 + (b % nbx) * 8, by0 = y0 + ((b / nbx) % nby) * 8, bz0 = z0 + (b / (nbx * nby)) * 8;
-    const int32_t c = threadIdx.x;
-    const int32_t lx = c & 7, ly = (c >> 3) & 7, lz = c >> 6;
-    const int32_t x = bx0 + lx, y = by0 + ly, z = bz0 + lz;
-    bool mine = (x < x0 + w) & (y < y0 + h) & (z < z0 + d);
-    if (sr >= 0) {
+// destroyVoxel and fixDepthField over the box of w x h x d voxels at
+// (x0, y0, z0) (inside the grid), in one pass: voxels with
+// (x-cx)^2+(y-cy)^2+(z-cz)^2 < cr^2 become -1 (cr <= 0: none), then the empty
+// ones within sr^2 of the centre (sr < 0: the whole box) are fixed, and every
+// voxel of the box goes to the render copy r (r.vox null: no copy).
+//
+// One workgroup of NT threads per tile of 32 x 8 x 8 voxels of the box.  A wave
+// reads a row of its surroundings with one load (64 voxels; only those within
+// reach) and makes the bitmap's row by a ballot, kEditRows rows in flight at
+// once; field_tile does the rest.
+// Workgroups of one launch may read a voxel that another has already carved
+// or fixed: it is not solid before or after (the carve test is applied to
+// what is read), and solid voxels outside the carve are never written.
+// Latency bound (launch, two or four rounds of loads, five barriers): eight
+// removeSpheres of radius 1-8 one after another 35 us (114 us when the device
+// was idle before), against 112 and 341 us for three launches each (carve,
+// per-voxel table scans over the box, copy of the box).
+constexpr int kEditY = 8, kEditZ = 8;
+constexpr int kEditRows = 25;
+template <int NT>
+__global__ void __launch_bounds__(NT) k_edit_box(GridDesc g, GridDesc r, FieldWords words, int32_t x0, int32_t y0,
+                                                 int32_t z0, int32_t w, int32_t h, int32_t d, uint32_t nbx,
+                                                 uint32_t nby, int32_t cx, int32_t cy, int32_t cz, int32_t sr,
+                                                 int32_t cr) {
+    using Tile = dev::FieldTile<kEditY, kEditZ>;
+    __shared__ Tile L;
+    const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t b = blockIdx.x;
+    // the tile's corner in the box and the extent of the box in the tile
+    const int32_t ox = (int32_t)(b % nbx) * 32, oy = (int32_t)((b / nbx) % nby) * kEditY,
+                  oz = (int32_t)(b / (nbx * nby)) * kEditZ;
+    const int32_t tw = w - ox < 32 ? w - ox : 32;
+    const int32_t bx = x0 + ox, by = y0 + oy, bz = z0 + oz;
+    auto dist2 = [&](int32_t x, int32_t y, int32_t z) {
         const int32_t ex = x - cx, ey = y - cy, ez = z - cz;
-        mine &= ex * ex + ey * ey + ez * ez < sr * sr;
+        return ex * ex + ey * ey + ez * ez;
+    };
+    auto carved = [&](int32_t x, int32_t y, int32_t z) { return cr > 0 && dist2(x, y, z) < cr * cr; };
+    // this thread's voxels: 32 along x, kCells rows apart in steps
+    constexpr int kCells = 32 * kEditY * kEditZ / NT;
+    const int32_t x = bx + (tid & 31);
+    int32_t was[kCells], old[kCells];
+    bool mine[kCells], fix = false;
+#pragma unroll
+    for (int j = 0; j < kCells; j++) {
+        const int32_t row = (tid >> 5) + j * (NT / 32);
+        const int32_t ly = row % kEditY, lz = row / kEditY;
+        mine[j] = ((tid & 31) < tw) & (oy + ly < h) & (oz + lz < d);
+        was[j] = mine[j] ? g.vox[(uint64_t)x + g.X * (uint64_t)(by + ly) + g.XY * (uint64_t)(bz + lz)] : 0;
     }
-    const uint64_t i = (uint64_t)x + g.X * (uint64_t)y + g.XY * (uint64_t)z;
-    const int32_t old = mine ? g.vox[i] : 0;
-    if (!__syncthreads_or(mine && old < 0)) return;  // nothing to fix in this brick
-    fill_rows_from_grid(g, rows, bx0, by0, bz0, c);
-    __syncthreads();
-    if (!mine || old >= 0) return;
-    const int32_t nv = scan_groups(rows, t, lx, ly, lz, old);
-    if (nv != old) g.vox[i] = nv;
+    // rows within 6 voxels of the tile, x from 16 before it
+    constexpr int kRows = Tile::SY * Tile::SZ, kWaves = NT / 64;
+    const int32_t gx = bx - 16 + lane;
+    const bool in_x = lane >= 10 && lane < 22 + tw && gx >= 0 && (uint32_t)gx < g.X;
+    for (int i0 = wave; i0 < kRows; i0 += kWaves * kEditRows) {
+        int32_t v[kEditRows];
+#pragma unroll
+        for (int j = 0; j < kEditRows; j++) {
+            const int32_t i = i0 + j * kWaves;
+            const int32_t gy = by - 6 + i % Tile::SY, gz = bz - 6 + i / Tile::SY;
+            v[j] = -1;
+            if (i < kRows && gy >= 0 && gz >= 0 && (uint32_t)gy < g.Y && (uint32_t)gz < g.Z && in_x)
+                v[j] = g.vox[(uint64_t)gx + g.X * (uint64_t)gy + g.XY * (uint64_t)gz];
+        }
+#pragma unroll
+        for (int j = 0; j < kEditRows; j++) {
+            const int32_t i = i0 + j * kWaves;
+            const uint64_t m = __ballot(v[j] >= 0 && !carved(gx, by - 6 + i % Tile::SY, bz - 6 + i / Tile::SY));
+            if (lane == 0 && i < kRows) L.s[i] = make_uint2((uint32_t)m, (uint32_t)(m >> 32));
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kCells; j++) {
+        const int32_t row = (tid >> 5) + j * (NT / 32);
+        const int32_t y = by + row % kEditY, z = bz + row / kEditY;
+        old[j] = mine[j] && carved(x, y, z) ? -1 : was[j];
+        fix |= mine[j] && old[j] < 0 && (sr < 0 || dist2(x, y, z) < sr * sr);
+    }
+    const bool any = __syncthreads_or(fix) != 0;
+    if (any) dev::field_tile<kEditY, kEditZ, NT>(L, tid, words);
+#pragma unroll
+    for (int j = 0; j < kCells; j++) {
+        if (!mine[j]) continue;
+        const int32_t row = (tid >> 5) + j * (NT / 32);
+        const int32_t y = by + row % kEditY, z = bz + row / kEditY;
+        int32_t now = old[j];
+        if (any && now < 0 && (sr < 0 || dist2(x, y, z) < sr * sr)) {
+            const uint32_t* p = L.plane + row * 6;
+            const uint32_t pl[5] = {p[0], p[1], p[2], p[3], p[4]};
+            if (!(p[5] >> (tid & 31) & 1u)) now = L.word[dev::level_at(pl, tid & 31)];
+        }
+        if (now != was[j]) g.vox[(uint64_t)x + g.X * (uint64_t)y + g.XY * (uint64_t)z] = now;
+        if (r.vox) r.vox[r.origin + (uint64_t)x + (uint64_t)r.SX * (uint64_t)y + r.SXY * (uint64_t)z] = now;
+    }
 }
 
-// destroyVoxel over the clipped box of removeSphere's first loop
-// (src/level.cpp:31-42): (x-cx)^2+(y-cy)^2+(z-cz)^2 < r^2.
-__global__ void __launch_bounds__(256) k_carve(GridDesc g, int32_t x0, int32_t y0, int32_t z0, int32_t w, int32_t h,
-                                                int32_t d, int32_t cx, int32_t cy, int32_t cz, int32_t r) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= (int64_t)w * h * d) return;
-    const int32_t x = x0 + (int32_t)(k % w);
-    const int32_t y = y0 + (int32_t)((k / w) % h);
-    const int32_t z = z0 + (int32_t)(k / ((int64_t)w * h));
-    const int32_t ex = x - cx, ey = y - cy, ez = z - cz;
-    if (ex * ex + ey * ey + ez * ez >= r * r) return;
-    g.vox[(uint64_t)x + g.X * (uint64_t)y + g.XY * (uint64_t)z] = -1;
-}
-
-__global__ void k_set_voxel(int32_t* vox, uint64_t i, int32_t v, int32_t* top, int32_t y) {
+// One voxel of the grid and of the render copy.
+__global__ void k_set_voxel(int32_t* vox, int32_t* copy, int32_t v, int32_t* top, int32_t y) {
     if (threadIdx.x == 0) {
-        vox[i] = v;
+        *vox = v;
+        *copy = v;
         if (v >= 0 && top) atomicMax(top, y);
     }
 }
@@ -345,21 +339,33 @@ inline void clip(int64_t& lo, int64_t& hi, int64_t n) {
 
 }  // namespace
 
-int launch_fix_depth_box(const GridDesc& g, const DepthTableDev& t, int32_t x0, int32_t y0, int32_t z0, int32_t x1,
-                         int32_t y1, int32_t z1, int32_t scx, int32_t scy, int32_t scz, int32_t sr, hipStream_t s) {
-    int64_t ax = x0, bx_ = x1, ay = y0, by_ = y1, az = z0, bz_ = z1;
-    clip(ax, bx_, g.X);
-    clip(ay, by_, g.Y);
-    clip(az, bz_, g.Z);
-    if (bx_ <= ax || by_ <= ay || bz_ <= az) return VRT_OK;
-    const int64_t w = bx_ - ax, h = by_ - ay, d = bz_ - az;
-    const int64_t nbx = (w + 7) / 8, nby = (h + 7) / 8, nbz = (d + 7) / 8;
-    const int64_t blocks = nbx * nby * nbz;
-    if (blocks > 0x7fffffff) return fail(VRT_ERR_INVALID, "box too large");
-    hipLaunchKernelGGL(k_fix_depth_box, dim3((uint32_t)blocks), dim3(512), 0, s, g, t, (int32_t)ax, (int32_t)ay,
-                       (int32_t)az, (int32_t)w, (int32_t)h, (int32_t)d, (int32_t)nbx, (int32_t)nby, scx, scy, scz,
-                       sr);
-    VRT_HIP(hipGetLastError());
+int launch_edit_box(const GridDesc& g, const GridDesc& render, const FieldWords& words, int64_t x0, int64_t y0,
+                    int64_t z0, int64_t x1, int64_t y1, int64_t z1, int32_t cx, int32_t cy, int32_t cz, int32_t sr,
+                    int32_t cr, hipStream_t s) {
+    clip(x0, x1, g.X);
+    clip(y0, y1, g.Y);
+    clip(z0, z1, g.Z);
+    if (x1 <= x0 || y1 <= y0 || z1 <= z0) return VRT_OK;
+    const int64_t w = x1 - x0, h = y1 - y0, d = z1 - z0;
+    const int64_t nbx = (w + 31) / 32, nby = (h + kEditY - 1) / kEditY, nbz = (d + kEditZ - 1) / kEditZ;
+    // An edit without a render copy is a server's, beside batches that fill the
+    // device: a workgroup of 512 threads waits there until some CU has two
+    // wave slots free on each SIMD (24 requests with 2 edits: 2801 us, with 256
+    // threads 2777).  On a device with room 512 threads are faster (above: 35
+    // and 114 us, with 256 threads 51 and 165).
+    const int threads = render.vox ? 512 : 256;
+    // a launch holds fewer than 2^32 threads: deep boxes go in slabs along z
+    const int64_t most = ((int64_t)1 << 32) / threads - 1;
+    if (nbx * nby > most) return fail(VRT_ERR_INVALID, "box too large");
+    const int64_t slab = most / (nbx * nby);
+    for (int64_t k = 0; k < nbz; k += slab) {
+        const dim3 blocks((uint32_t)(nbx * nby * std::min(slab, nbz - k)));
+        auto* kernel = render.vox ? k_edit_box<512> : k_edit_box<256>;
+        hipLaunchKernelGGL(kernel, blocks, dim3(threads), 0, s, g, render, words, (int32_t)x0, (int32_t)y0,
+                           (int32_t)(z0 + k * kEditZ), (int32_t)w, (int32_t)h, (int32_t)(d - k * kEditZ),
+                           (uint32_t)nbx, (uint32_t)nby, cx, cy, cz, sr, cr);
+        VRT_HIP(hipGetLastError());
+    }
     return VRT_OK;
 }
 
@@ -382,26 +388,14 @@ int launch_build_depth_field(const GridDesc& g, const GridDesc& render, const Fi
     return VRT_OK;
 }
 
-int launch_carve_sphere(const GridDesc& g, int32_t cx, int32_t cy, int32_t cz, int32_t r, hipStream_t s) {
-    if (r <= 0) return VRT_OK;
-    int64_t ax = (int64_t)cx - r, bx_ = (int64_t)cx + r, ay = (int64_t)cy - r, by_ = (int64_t)cy + r,
-            az = (int64_t)cz - r, bz_ = (int64_t)cz + r;
-    clip(ax, bx_, g.X);
-    clip(ay, by_, g.Y);
-    clip(az, bz_, g.Z);
-    if (bx_ <= ax || by_ <= ay || bz_ <= az) return VRT_OK;
-    const int64_t w = bx_ - ax, h = by_ - ay, d = bz_ - az;
-    const int64_t blocks = (w * h * d + 255) / 256;
-    if (blocks > 0x7fffffff) return fail(VRT_ERR_INVALID, "sphere too large");
-    hipLaunchKernelGGL(k_carve, dim3((uint32_t)blocks), dim3(256), 0, s, g, (int32_t)ax, (int32_t)ay, (int32_t)az,
-                       (int32_t)w, (int32_t)h, (int32_t)d, cx, cy, cz, r);
-    VRT_HIP(hipGetLastError());
-    return VRT_OK;
-}
-
-int launch_set_voxel(const GridDesc& g, int64_t index, int32_t y, int32_t v, hipStream_t s) {
-    if (index < 0 || (uint64_t)index >= g.count) return fail(VRT_ERR_INVALID, "voxel index out of range");
-    hipLaunchKernelGGL(k_set_voxel, dim3(1), dim3(64), 0, s, g.vox, (uint64_t)index, v, g.top, y);
+int launch_set_voxel(const GridDesc& g, const GridDesc& render, int32_t x, int32_t y, int32_t z, int32_t v,
+                     hipStream_t s) {
+    if (x < 0 || y < 0 || z < 0 || (uint32_t)x >= g.X || (uint32_t)y >= g.Y || (uint32_t)z >= g.Z)
+        return fail(VRT_ERR_INVALID, "voxel out of range");
+    auto at = [&](const GridDesc& d) {
+        return d.vox + (d.origin + (uint64_t)x + (uint64_t)d.SX * (uint64_t)y + d.SXY * (uint64_t)z);
+    };
+    hipLaunchKernelGGL(k_set_voxel, dim3(1), dim3(64), 0, s, at(g), at(render), v, g.top, y);
     VRT_HIP(hipGetLastError());
     return VRT_OK;
 }

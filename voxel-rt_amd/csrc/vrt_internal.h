@@ -126,19 +126,6 @@ struct FieldWords {
     int32_t word[kFieldLevels + 2];
 };
 
-struct DepthTableDev {
-    const int32_t* packed;  // (dx+8) | (dy+8)<<5 | (dz+8)<<10, sorted by dist descending
-    const float* dist;      // dist of each packed entry
-    int32_t n;              // entries with dist > -6
-    int32_t n_near;         // leading entries with dist > -2
-    // The same entries grouped into rows: one per (distance, dy, dz), in the
-    // same order of distance, with the mask of their dx (bit dx+7).
-    const int32_t* rows;      // mask | (dy+8)<<16 | (dz+8)<<21
-    const float* rows_dist;   // dist of each row
-    int32_t n_rows;           // rows with dist > -6
-    int32_t n_rows_near;      // leading rows with dist > -2
-};
-
 struct Ctx;
 
 // ---- kernels launch wrappers (vrt_render.hip / vrt_edit.hip / vrt_world.hip)
@@ -166,17 +153,22 @@ int selftest_division(uint32_t d_begin, uint32_t d_count, unsigned long long* ba
 int selftest_reciprocal(uint64_t first, uint64_t count, unsigned long long* bad_dev, hipStream_t s);
 int batch_occupancy(const vrt_batch_config& cfg, int32_t* waves_per_cu);
 
-int launch_fix_depth_box(const GridDesc& g, const DepthTableDev& t, int32_t x0, int32_t y0, int32_t z0,
-                         int32_t x1, int32_t y1, int32_t z1, int32_t sphere_cx, int32_t sphere_cy,
-                         int32_t sphere_cz, int32_t sphere_r, hipStream_t s);
+// destroyVoxel within cr of (cx, cy, cz) (cr <= 0: none), then fixDepthField
+// within sr of it (sr < 0: everywhere), over the voxels of the box [x0,x1) x
+// [y0,y1) x [z0,z1) (clipped to the grid); the box goes to `render` too unless
+// render.vox is null.  cr <= sr where both apply.
+int launch_edit_box(const GridDesc& g, const GridDesc& render, const FieldWords& words, int64_t x0, int64_t y0,
+                    int64_t z0, int64_t x1, int64_t y1, int64_t z1, int32_t cx, int32_t cy, int32_t cz, int32_t sr,
+                    int32_t cr, hipStream_t s);
 // Whole-grid depth field: solidity bitmap (Y*Z rows of solid_bits_words(g)
 // words), then every tile's words into the grid and into `render`, the
 // padded copy of the whole grid.
 uint32_t solid_bits_words(const GridDesc& g);
 int launch_build_depth_field(const GridDesc& g, const GridDesc& render, const FieldWords& words, uint32_t* bits,
                              hipStream_t s);
-int launch_carve_sphere(const GridDesc& g, int32_t cx, int32_t cy, int32_t cz, int32_t r, hipStream_t s);
-int launch_set_voxel(const GridDesc& g, int64_t index, int32_t y, int32_t v, hipStream_t s);
+// One voxel of the grid and of the render copy; raises *g.top for a solid one.
+int launch_set_voxel(const GridDesc& g, const GridDesc& render, int32_t x, int32_t y, int32_t z, int32_t v,
+                     hipStream_t s);
 // Raises *g.top to the highest y with a solid voxel in the box [x0,x1) x
 // [y0,y1) x [z0,z1) (clipped to the grid); with reset, sets it to -1 first.
 int launch_solid_top(const GridDesc& g, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1,
@@ -221,11 +213,6 @@ struct vrt_ctx {
     unsigned long long* parts = nullptr;     // plain draws' partial counts (kPartsCap entries)
     int64_t parts_used = 0;                  // entries not yet folded into `counters`
     uint64_t draws = 0;
-    int32_t* table_packed = nullptr;
-    float* table_dist = nullptr;
-    int32_t* table_rows = nullptr;
-    float* table_rows_dist = nullptr;
-    vrt::DepthTableDev table{};
     vrt::FieldWords words{};
     uint32_t* solid_bits = nullptr;  // whole-grid build scratch, allocated by the first build
     int32_t num_cus = 0;
@@ -250,14 +237,12 @@ int solid_top_full(vrt_ctx* c);  // recomputes *grid.top over the whole grid
 // grid into the render copy, on the context's stream.
 int refresh_render(vrt_ctx* c, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1);
 int refresh_render_all(vrt_ctx* c);
-int refresh_render_on(vrt_ctx* c, hipStream_t s, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1,
-                      int64_t z1);
-// removeSphere in two parts on stream s: the carve and depth-field repair of
-// the grid (render kernels never read it), then the copy of the edited box
-// into the render copy (what in-flight renders must not see).
-int remove_sphere_grid(vrt_ctx* c, int32_t cx, int32_t cy, int32_t cz, int32_t radius, hipStream_t s);
-int remove_sphere_refresh(vrt_ctx* c, int32_t cx, int32_t cy, int32_t cz, int32_t radius, hipStream_t s);
-// The same two refreshes into another copy laid out like the render copy.
+// removeSphere on stream s: carve and depth-field repair of the grid and, unless
+// render.vox is null, of the edited box of that padded copy.
+int remove_sphere_on(vrt_ctx* c, const GridDesc& render, int32_t cx, int32_t cy, int32_t cz, int32_t radius,
+                     hipStream_t s);
+// The same refresh, and that of a removeSphere's box, into another copy laid
+// out like the render copy.
 int refresh_copy_on(vrt_ctx* c, const GridDesc& dst, hipStream_t s, int64_t x0, int64_t y0, int64_t z0, int64_t x1,
                     int64_t y1, int64_t z1);
 int remove_sphere_refresh_into(vrt_ctx* c, const GridDesc& dst, int32_t cx, int32_t cy, int32_t cz, int32_t radius,

@@ -250,7 +250,9 @@ int catch_up(vrt_server* s, int32_t k) {
 int apply_edit(vrt_server* s, const Item& it) {
     vrt_ctx* c = s->ctx;
     // carve + repair of the grid: no render reads it, so no wait
-    if (int rc = remove_sphere_grid(c, it.cx, it.cy, it.cz, it.r, s->edit_stream)) return rc;
+    GridDesc none = c->rgrid;
+    none.vox = nullptr;
+    if (int rc = remove_sphere_on(c, none, it.cx, it.cy, it.cz, it.r, s->edit_stream)) return rc;
     s->version_applied++;
     s->recent.push_back({s->version_applied, it.cx, it.cy, it.cz, it.r});
     if (int rc = catch_up(s, (int32_t)(s->version_applied & 1))) return rc;
