@@ -109,3 +109,32 @@ def test_fix_box_equals_oracle(gpu, orc, lo, hi):
     assert np.array_equal(got, ref), "%d voxels differ" % int((got != ref).sum())
     check_rays(gpu, orc, ctx, ref, dims, rng)
     ctx.close()
+
+
+@pytest.mark.parametrize("lo,size", [((3, 2, 1), (1, 1, 1)), ((0, 0, 0), (10, 10, 10)), ((255, 30, 190), (1, 70, 60)),
+                                     ((0, 0, 0), (256, 64, 16)), ((0, 0, 0), (256, 64, 32)), ((1, 0, 3), (255, 90, 77)),
+                                     ((0, 0, 0), (256, 129, 250))])
+def test_region_upload_in_pieces(gpu, orc, lo, size):
+    """Partial uploads of less than, exactly and more than the staging's pieces
+    (2^18 words), pieces that end inside a row; the solid top follows."""
+    dims = (256, 130, 251)
+    rng = np.random.default_rng(size[0] + size[1])
+    ctx = gpu.Context(dims)
+    host = random_world(rng, dims, 0.01)
+    hi = tuple(lo[k] + size[k] - (k == 0) for k in range(3))  # inside the grid, or the corners would be swapped
+    ctx.upload_region(host, lo, hi)
+    ref = np.full_like(host, -1)
+    box = tuple(slice(lo[k], lo[k] + size[k]) for k in (2, 1, 0))
+    ref.reshape(dims[::-1])[box] = host.reshape(dims[::-1])[box]
+    got = ctx.download()
+    assert np.array_equal(got, ref), "%d voxels differ" % int((got != ref).sum())
+    check_rays(gpu, orc, ctx, ref, dims, rng)
+    # rays that rise take the cutoff at the solid top when no steps are asked for
+    n = 4000
+    start = np.stack([rng.uniform(0, d, n) for d in dims], 1).astype(np.float32)
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    d[:, 1] = np.abs(d[:, 1])
+    dist = np.full(n, 300, np.int32)
+    g, r = ctx.cast_rays(start, d, dist, 384, steps=False), orc.cast_rays(ref, dims, start, d, dist, 384)
+    assert np.array_equal(g["hit"], r["hit"])
+    ctx.close()

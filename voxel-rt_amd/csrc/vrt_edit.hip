@@ -268,6 +268,22 @@ __global__ void k_set_voxel(int32_t* vox, int32_t* copy, int32_t v, int32_t* top
     }
 }
 
+// Words [first, first + n) of the box of nx x ny x ... voxels at (x0, y0, z0),
+// x fastest, from `src` (pinned host memory, read over the link) into the grid
+// and the render copy; `top`: the highest y of a solid voxel among them.
+__global__ void __launch_bounds__(256) k_put_box(GridDesc g, GridDesc r, const int32_t* __restrict__ src,
+                                                 uint64_t first, uint32_t n, uint32_t nx, uint32_t ny, uint32_t x0,
+                                                 uint32_t y0, uint32_t z0, int32_t top) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i == 0 && top > *g.top) *g.top = top;
+    if (i >= n) return;
+    const int32_t v = src[i];
+    const uint64_t k = first + i, row = k / nx;
+    const uint64_t x = x0 + k % nx, y = y0 + row % ny, z = z0 + row / ny;
+    g.vox[x + g.X * y + g.XY * z] = v;
+    r.vox[r.origin + x + (uint64_t)r.SX * y + r.SXY * z] = v;
+}
+
 __global__ void k_set_word(int32_t* p, int32_t v) {
     if (threadIdx.x == 0) *p = v;
 }
@@ -396,6 +412,16 @@ int launch_set_voxel(const GridDesc& g, const GridDesc& render, int32_t x, int32
         return d.vox + (d.origin + (uint64_t)x + (uint64_t)d.SX * (uint64_t)y + d.SXY * (uint64_t)z);
     };
     hipLaunchKernelGGL(k_set_voxel, dim3(1), dim3(64), 0, s, at(g), at(render), v, g.top, y);
+    VRT_HIP(hipGetLastError());
+    return VRT_OK;
+}
+
+int launch_put_box(const GridDesc& g, const GridDesc& render, const int32_t* src, int64_t first, int64_t n, int64_t nx,
+                   int64_t ny, int64_t x0, int64_t y0, int64_t z0, int32_t top, hipStream_t s) {
+    if (n <= 0) return VRT_OK;
+    if (n > 0x7fffffff) return fail(VRT_ERR_INVALID, "too many words in one piece");
+    hipLaunchKernelGGL(k_put_box, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, g, render, src, (uint64_t)first,
+                       (uint32_t)n, (uint32_t)nx, (uint32_t)ny, (uint32_t)x0, (uint32_t)y0, (uint32_t)z0, top);
     VRT_HIP(hipGetLastError());
     return VRT_OK;
 }

@@ -126,6 +126,9 @@ struct FieldWords {
     int32_t word[kFieldLevels + 2];
 };
 
+// Words of one of the two pieces of a context's upload staging (1 MiB).
+constexpr int64_t kStagePiece = (int64_t)1 << 18;
+
 struct Ctx;
 
 // ---- kernels launch wrappers (vrt_render.hip / vrt_edit.hip / vrt_world.hip)
@@ -169,6 +172,11 @@ int launch_build_depth_field(const GridDesc& g, const GridDesc& render, const Fi
 // One voxel of the grid and of the render copy; raises *g.top for a solid one.
 int launch_set_voxel(const GridDesc& g, const GridDesc& render, int32_t x, int32_t y, int32_t z, int32_t v,
                      hipStream_t s);
+// Words [first, first + n) of the box at (x0, y0, z0), nx x ny voxels per z,
+// from pinned host memory into the grid and the render copy; raises *g.top to
+// `top`.
+int launch_put_box(const GridDesc& g, const GridDesc& render, const int32_t* src, int64_t first, int64_t n, int64_t nx,
+                   int64_t ny, int64_t x0, int64_t y0, int64_t z0, int32_t top, hipStream_t s);
 // Raises *g.top to the highest y with a solid voxel in the box [x0,x1) x
 // [y0,y1) x [z0,z1) (clipped to the grid); with reset, sets it to -1 first.
 int launch_solid_top(const GridDesc& g, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1,
@@ -215,6 +223,10 @@ struct vrt_ctx {
     uint64_t draws = 0;
     vrt::FieldWords words{};
     uint32_t* solid_bits = nullptr;  // whole-grid build scratch, allocated by the first build
+    // Pinned staging of small partial uploads, two pieces of kStagePiece words,
+    // allocated by the first one; no upload leaves work on it when it returns.
+    int32_t* stage = nullptr;
+    hipEvent_t stage_done[2] = {nullptr, nullptr};
     int32_t num_cus = 0;
     bool tuned = false;
     vrt_batch_config tuned_cfg{8, 8, 0, 0};
