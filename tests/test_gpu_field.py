@@ -138,3 +138,25 @@ def test_region_upload_in_pieces(gpu, orc, lo, size):
     g, r = ctx.cast_rays(start, d, dist, 384, steps=False), orc.cast_rays(ref, dims, start, d, dist, 384)
     assert np.array_equal(g["hit"], r["hit"])
     ctx.close()
+
+
+@pytest.mark.parametrize("dims", DIMS, ids=["%dx%dx%d" % d for d in DIMS])
+def test_device_upload_at_odd_sizes(gpu, orc, dims):
+    """vrt_upload_device: grid, render copy and solid top in one pass, rows of
+    every length modulo four and grids of few rows."""
+    rng = np.random.default_rng(sum(dims))
+    world = random_world(rng, dims, 0.02)
+    ctx = gpu.Context(dims)
+    buf = gpu.DeviceBuffer(world.nbytes)
+    buf.upload(world)
+    gpu.call("vrt_upload_device", ctx.h, buf.addr)
+    assert np.array_equal(ctx.download(), world)
+    check_rays(gpu, orc, ctx, world, dims, rng)
+    n = 2000
+    start = np.stack([rng.uniform(0, d, n) for d in dims], 1).astype(np.float32)
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    d[:, 1] = np.abs(d[:, 1])
+    dist = np.full(n, 300, np.int32)
+    g, r = ctx.cast_rays(start, d, dist, 384, steps=False), orc.cast_rays(world, dims, start, d, dist, 384)
+    assert np.array_equal(g["hit"], r["hit"])
+    ctx.close()

@@ -275,10 +275,6 @@ int read_top(vrt_ctx* c) {
     return VRT_OK;
 }
 
-int solid_top_full(vrt_ctx* c) {
-    return launch_solid_top(c->grid, 0, 0, 0, c->grid.X, c->grid.Y, c->grid.Z, true, c->stream);
-}
-
 int refresh_render(vrt_ctx* c, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1) {
     return refresh_copy_on(c, c->rgrid, c->stream, x0, y0, z0, x1, y1, z1);
 }
@@ -318,8 +314,6 @@ int remove_sphere_refresh_into(vrt_ctx* c, const GridDesc& dst, int32_t cx, int3
     return refresh_copy_on(c, dst, s, (int64_t)cx - M, (int64_t)cy - M, (int64_t)cz - M, (int64_t)cx + M,
                            (int64_t)cy + M, (int64_t)cz + M);
 }
-
-int refresh_render_all(vrt_ctx* c) { return refresh_render(c, 0, 0, 0, c->grid.X, c->grid.Y, c->grid.Z); }
 
 }  // namespace vrt
 
@@ -404,9 +398,7 @@ int vrt_create(vrt_ctx** out, int64_t X, int64_t Y, int64_t Z, int32_t device) {
         return bail(hip_fail(e, "hipMemsetAsync"));
     rc = launch_fill(c->grid.vox, count, -1, c->stream);
     if (!rc) rc = launch_fill(c->rgrid.vox, c->rgrid.count, kGuardValue, c->stream);
-    if (!rc) rc = refresh_render_all(c);
-    if (rc) return bail(rc);
-    rc = launch_solid_top(c->grid, 0, 0, 0, 0, 0, 0, true, c->stream);  // no solid voxel yet: -1
+    if (!rc) rc = launch_load_grid(c->grid, c->rgrid, c->grid.vox, c->stream);
     if (rc) return bail(rc);
     c->top_host = -1;
     if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return bail(hip_fail(e, "hipStreamSynchronize"));
@@ -466,24 +458,20 @@ int vrt_upload(vrt_ctx* ctx, const int32_t* host_voxels) {
     if (!host_voxels) return fail(VRT_ERR_INVALID, "null voxels");
     VRT_HIP(hipMemcpyAsync(ctx->grid.vox, host_voxels, ctx->grid.count * sizeof(int32_t), hipMemcpyHostToDevice,
                            ctx->stream));
-    if (int rc = solid_top_full(ctx)) return rc;
-    if (int rc = refresh_render_all(ctx)) return rc;
+    if (int rc = launch_load_grid(ctx->grid, ctx->rgrid, ctx->grid.vox, ctx->stream)) return rc;
     return read_top(ctx);
 }
 
 int vrt_upload_device(vrt_ctx* ctx, const int32_t* device_voxels) {
     if (int rc = check_ctx(ctx)) return rc;
     if (!device_voxels) return fail(VRT_ERR_INVALID, "null voxels");
-    if (int rc = launch_copy(ctx->grid.vox, device_voxels, ctx->grid.count, ctx->stream)) return rc;
-    if (int rc = solid_top_full(ctx)) return rc;
-    if (int rc = refresh_render_all(ctx)) return rc;
+    if (int rc = launch_load_grid(ctx->grid, ctx->rgrid, device_voxels, ctx->stream)) return rc;
     return read_top(ctx);
 }
 
 int vrt_grid_modified(vrt_ctx* ctx) {
     if (int rc = check_ctx(ctx)) return rc;
-    if (int rc = solid_top_full(ctx)) return rc;
-    if (int rc = refresh_render_all(ctx)) return rc;
+    if (int rc = launch_load_grid(ctx->grid, ctx->rgrid, ctx->grid.vox, ctx->stream)) return rc;
     return read_top(ctx);
 }
 
@@ -662,7 +650,7 @@ int vrt_upload_region_f(vrt_ctx* ctx, const int32_t* host_voxels, const float st
         y_lo = (lo % (int64_t)g.XY) / g.X;
         y_hi = ((hi - 1) % (int64_t)g.XY) / g.X + 1;
     }
-    if (int rc = launch_solid_top(g, 0, y_lo, z_lo, g.X, y_hi, z_hi, false, ctx->stream)) return rc;
+    if (int rc = launch_solid_top(g, 0, y_lo, z_lo, g.X, y_hi, z_hi, ctx->stream)) return rc;
     if (int rc = refresh_render(ctx, 0, y_lo, z_lo, g.X, y_hi, z_hi)) return rc;
     return read_top(ctx);
 }
@@ -930,8 +918,7 @@ int vrt_world_generate_device(vrt_ctx* ctx, const vrt_world_params* p) {
     if (int rc = check_ctx(ctx)) return rc;
     if (!p) return fail(VRT_ERR_INVALID, "null params");
     if (int rc = world_generate_device(ctx->grid, *p, ctx->stream)) return rc;
-    if (int rc = solid_top_full(ctx)) return rc;
-    if (int rc = refresh_render_all(ctx)) return rc;
+    if (int rc = launch_load_grid(ctx->grid, ctx->rgrid, ctx->grid.vox, ctx->stream)) return rc;
     return read_top(ctx);
 }
 

@@ -62,60 +62,84 @@ __global__ void __launch_bounds__(256) k_solid_bits(GridDesc g, uint32_t* __rest
     }
 }
 
-// Whole-grid build: one workgroup per tile of 32 x 8 x 16 voxels, whose
-// distances come from the bitmap (field_tile).  Tiles without a solid voxel in
-// reach take -6 and tiles of solid voxels keep their words, both without that
-// work.  The tile's words go to the grid and, with the words that are kept, to
-// the padded render copy, so the copy needs no pass of its own; only words
-// that are kept are read.  Workgroup b runs on XCD b mod 8 and takes the tiles
-// of that eighth of the grid, so a tile's neighbours share the L2 that holds
-// the bitmap's rows and the copy's lines between two tiles.
-// 1024x256x1024 (1 GiB): 0.90 ms, against 7.18 ms for a table scan per voxel
-// plus 0.09 ms of brick flags and 0.38 ms of copying to the render copy; the
-// memory it must move (the copy and the changed words written, the kept ones
-// read, 2.1 GB) takes 0.45 ms at the rate of a large copy.
-constexpr int kTileY = 8, kTileZ = 16, kTileThreads = kTileY * kTileZ;
+// Whole-grid build: one workgroup per kTileRun tiles of 32 x 8 x 16 voxels side
+// by side in x, whose distances come from the bitmap (field_tile), one tile
+// after the other.  Tiles without a solid voxel in reach take -6 and tiles of
+// solid voxels keep their words, both without that work.  The words then go to
+// the grid and, with the words that are kept, to the padded render copy, so the
+// copy needs no pass of its own; only words that are kept are read.
+//
+// Bound by memory, the writes above all.  1024x256x1024 (1 GiB): 0.68 ms, where
+// a table scan per voxel took 7.18 ms and 0.38 ms more to copy the grid; the
+// 2.1 GB that it must move take 0.45 ms at the rate of a large copy.  The
+// copy's rows start anywhere in a 128-byte line, so a run's two ends write
+// parts of lines: runs of one tile (128 bytes) took 0.81 ms.  (Rows padded to
+// whole lines gained 5% there and cost 1% of every frame.)  Workgroup b runs on
+// XCD b mod 8 and takes the tiles of that eighth of the grid, so neighbours
+// share the L2 that holds the bitmap's rows and the lines between two runs:
+// writing such runs without that order took twice as long.
+constexpr int kTileY = 8, kTileZ = 16, kTileThreads = kTileY * kTileZ, kTileRun = 4;
 __global__ void __launch_bounds__(kTileThreads) k_field_tiles(GridDesc g, GridDesc r, FieldWords words,
                                                               const uint32_t* __restrict__ bits, uint32_t W,
-                                                              uint32_t nx, uint32_t ny, uint32_t tiles) {
+                                                              uint32_t runs, uint32_t ny, uint32_t total) {
     using Tile = dev::FieldTile<kTileY, kTileZ>;
     __shared__ Tile L;
-    const uint32_t tile = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-    if (tile >= tiles) return;
+    __shared__ uint32_t planes[kTileRun][kTileThreads * 6];
+    __shared__ int32_t word[kFieldLevels + 2];
+    const uint32_t run = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    if (run >= total) return;
     const int32_t tid = threadIdx.x;
-    const uint32_t kx = tile % nx;
-    const int32_t x0 = (int32_t)(kx * 32), y0 = (int32_t)((tile / nx) % ny) * kTileY,
-                  z0 = (int32_t)(tile / (nx * ny)) * kTileZ;
-    bool any = false, full = true;
-    for (int32_t i = tid; i < Tile::SZ * Tile::SY; i += kTileThreads) {
-        const int32_t y = i % Tile::SY - 6, z = i / Tile::SY - 6;
-        const int64_t gy = (int64_t)y0 + y, gz = (int64_t)z0 + z;
-        uint2 v = make_uint2(0, 0);
-        if (gy >= 0 && gz >= 0 && gy < (int64_t)g.Y && gz < (int64_t)g.Z) {
-            const uint32_t* rw = bits + ((uint64_t)gy + (uint64_t)g.Y * (uint64_t)gz) * W + kx;
-            v = make_uint2(rw[0], rw[1]);
-        }
-        L.s[i] = v;
-        any |= (v.x | v.y) != 0u;
-        if (y >= 0 && y < kTileY && z >= 0 && z < kTileZ) full &= dev::funnel(v.y, v.x, 16) == 0xffffffffu;
-    }
-    any = __syncthreads_or(any) != 0;
-    full = any && __syncthreads_and(full) != 0;
-    if (any && !full) {
-        dev::field_tile<kTileY, kTileZ, kTileThreads>(L, tid, words);
-    } else {
-        if (tid < kFieldLevels + 2) L.word[tid] = words.word[tid];
-        uint32_t* p = L.plane + tid * 6;
+    const uint32_t k0 = (run % runs) * kTileRun;  // the run's first bitmap word
+    const int32_t y0 = (int32_t)((run / runs) % ny) * kTileY, z0 = (int32_t)(run / (runs * ny)) * kTileZ;
+    const int32_t tiles = (int32_t)min((uint32_t)kTileRun, W - 1 - k0);
+    if (tid < kFieldLevels + 2) word[tid] = words.word[tid];
+    // bitmap rows of a tile, two words each, kRowSteps rows per thread
+    constexpr int kRowSteps = (Tile::SZ * Tile::SY + kTileThreads - 1) / kTileThreads;
+    uint2 rows[kRowSteps];
+    auto load_rows = [&](int32_t t) {
 #pragma unroll
-        for (int k = 0; k < 5; k++) p[k] = !full && ((kFieldLevels + 1) >> k & 1) ? 0xffffffffu : 0u;
-        p[5] = full ? 0xffffffffu : 0u;
-        __syncthreads();
+        for (int j = 0; j < kRowSteps; j++) {
+            const int32_t i = tid + j * kTileThreads;
+            const int32_t gy = y0 - 6 + i % Tile::SY, gz = z0 - 6 + i / Tile::SY;
+            rows[j] = make_uint2(0, 0);
+            if (i < Tile::SZ * Tile::SY && gy >= 0 && gz >= 0 && (uint32_t)gy < g.Y && (uint32_t)gz < g.Z) {
+                const uint32_t* rw = bits + ((uint64_t)gy + (uint64_t)g.Y * (uint64_t)gz) * W + k0 + t;
+                rows[j] = make_uint2(rw[0], rw[1]);
+            }
+        }
+    };
+    load_rows(0);
+    for (int32_t t = 0; t < tiles; t++) {
+        bool any = false, full = true;
+#pragma unroll
+        for (int j = 0; j < kRowSteps; j++) {
+            const int32_t i = tid + j * kTileThreads;
+            const int32_t y = i % Tile::SY - 6, z = i / Tile::SY - 6;
+            if (i >= Tile::SZ * Tile::SY) continue;
+            L.s[i] = rows[j];
+            any |= (rows[j].x | rows[j].y) != 0u;
+            if (y >= 0 && y < kTileY && z >= 0 && z < kTileZ)
+                full &= dev::funnel(rows[j].y, rows[j].x, 16) == 0xffffffffu;
+        }
+        if (t + 1 < tiles) load_rows(t + 1);  // in flight during this tile's work
+        any = __syncthreads_or(any) != 0;
+        full = any && __syncthreads_and(full) != 0;
+        if (any && !full) {
+            dev::field_tile<kTileY, kTileZ, kTileThreads>(L, planes[t], tid);
+        } else {
+            uint32_t* p = planes[t] + tid * 6;
+#pragma unroll
+            for (int k = 0; k < 5; k++) p[k] = !full && ((kFieldLevels + 1) >> k & 1) ? 0xffffffffu : 0u;
+            p[5] = full ? 0xffffffffu : 0u;
+            __syncthreads();
+        }
     }
-    // four voxels per lane and step, eight lanes per row: 128 bytes of a row
-    constexpr int kSteps = 8;
-    dev::vox4 v[kSteps];
-    const int32_t quad = tid & 7, x = x0 + 4 * quad;
-    auto row_of = [&](int j) { return j * (kTileThreads / 8) + (tid >> 3); };
+    // four voxels per lane, the run's lanes side by side: 512 bytes of a row
+    constexpr int kLanes = 8 * kTileRun, kSteps = 8;
+    const int32_t lane = tid % kLanes, x = (int32_t)(k0 * 32) + 4 * lane;
+    if (lane >= 8 * tiles || (int64_t)x >= (int64_t)g.X) return;
+    const uint32_t* plane = planes[lane / 8];
+    const uint32_t b = 4 * (lane % 8);
     auto cell = [&](const GridDesc& d, int row) {
         return d.origin + (uint64_t)x + (uint64_t)d.SX * (uint64_t)(y0 + row % kTileY) +
                d.SXY * (uint64_t)(z0 + row / kTileY);
@@ -123,41 +147,42 @@ __global__ void __launch_bounds__(kTileThreads) k_field_tiles(GridDesc g, GridDe
     auto inside = [&](int row) {
         return (uint32_t)(y0 + row % kTileY) < g.Y && (uint32_t)(z0 + row / kTileY) < g.Z;
     };
-    if ((int64_t)x + 3 < (int64_t)g.X) {
+    for (int row0 = tid / kLanes; row0 < Tile::kRows; row0 += kSteps * (kTileThreads / kLanes)) {
+        if ((int64_t)x + 3 < (int64_t)g.X) {
+            dev::vox4 v[kSteps];
 #pragma unroll
-        for (int j = 0; j < kSteps; j++) {
-            const int row = row_of(j);
-            if (inside(row) && ((L.plane[row * 6 + 5] >> (4 * quad)) & 15u))
-                v[j] = *(const dev::vox4*)(g.vox + cell(g, row));
-        }
+            for (int j = 0; j < kSteps; j++) {
+                const int row = row0 + j * (kTileThreads / kLanes);
+                if (inside(row) && ((plane[row * 6 + 5] >> b) & 15u)) v[j] = *(const dev::vox4*)(g.vox + cell(g, row));
+            }
 #pragma unroll
-        for (int j = 0; j < kSteps; j++) {
-            const int row = row_of(j);
-            if (!inside(row)) continue;
-            const uint32_t* p = L.plane + row * 6;
-            const uint32_t b = 4 * quad, keep = (p[5] >> b) & 15u;
-            const uint32_t pl[5] = {p[0], p[1], p[2], p[3], p[4]};
-            dev::vox4 o;
-            o.x = keep & 1u ? v[j].x : L.word[dev::level_at(pl, b)];
-            o.y = keep & 2u ? v[j].y : L.word[dev::level_at(pl, b + 1)];
-            o.z = keep & 4u ? v[j].z : L.word[dev::level_at(pl, b + 2)];
-            o.w = keep & 8u ? v[j].w : L.word[dev::level_at(pl, b + 3)];
-            if (keep != 15u) *(dev::vox4*)(g.vox + cell(g, row)) = o;
-            *(dev::vox4*)(r.vox + cell(r, row)) = o;
-        }
-    } else {
-        for (int j = 0; j < kSteps; j++) {
-            const int row = row_of(j);
-            if (!inside(row)) continue;
-            const uint32_t* p = L.plane + row * 6;
-            const uint32_t pl[5] = {p[0], p[1], p[2], p[3], p[4]};
-            for (int k = 0; k < 4 && (int64_t)x + k < (int64_t)g.X; k++) {
-                const uint32_t b = 4 * quad + k;
-                int32_t* w = g.vox + cell(g, row) + k;
-                int32_t o;
-                if (p[5] >> b & 1u) o = *w;
-                else *w = o = L.word[dev::level_at(pl, b)];
-                r.vox[cell(r, row) + k] = o;
+            for (int j = 0; j < kSteps; j++) {
+                const int row = row0 + j * (kTileThreads / kLanes);
+                if (!inside(row)) continue;
+                const uint32_t* p = plane + row * 6;
+                const uint32_t keep = (p[5] >> b) & 15u;
+                const uint32_t pl[5] = {p[0], p[1], p[2], p[3], p[4]};
+                dev::vox4 o;
+                o.x = keep & 1u ? v[j].x : word[dev::level_at(pl, b)];
+                o.y = keep & 2u ? v[j].y : word[dev::level_at(pl, b + 1)];
+                o.z = keep & 4u ? v[j].z : word[dev::level_at(pl, b + 2)];
+                o.w = keep & 8u ? v[j].w : word[dev::level_at(pl, b + 3)];
+                if (keep != 15u) *(dev::vox4*)(g.vox + cell(g, row)) = o;
+                *(dev::vox4*)(r.vox + cell(r, row)) = o;
+            }
+        } else {
+            for (int j = 0; j < kSteps; j++) {
+                const int row = row0 + j * (kTileThreads / kLanes);
+                if (!inside(row)) continue;
+                const uint32_t* p = plane + row * 6;
+                const uint32_t pl[5] = {p[0], p[1], p[2], p[3], p[4]};
+                for (int k = 0; k < 4 && (int64_t)x + k < (int64_t)g.X; k++) {
+                    int32_t* w = g.vox + cell(g, row) + k;
+                    int32_t o;
+                    if (p[5] >> (b + k) & 1u) o = *w;
+                    else *w = o = word[dev::level_at(pl, b + k)];
+                    r.vox[cell(r, row) + k] = o;
+                }
             }
         }
     }
@@ -189,7 +214,9 @@ __global__ void __launch_bounds__(NT) k_edit_box(GridDesc g, GridDesc r, FieldWo
                                                  int32_t cr) {
     using Tile = dev::FieldTile<kEditY, kEditZ>;
     __shared__ Tile L;
+    __shared__ int32_t word[kFieldLevels + 2];
     const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid < kFieldLevels + 2) word[tid] = words.word[tid];
     const uint32_t b = blockIdx.x;
     // the tile's corner in the box and the extent of the box in the tile
     const int32_t ox = (int32_t)(b % nbx) * 32, oy = (int32_t)((b / nbx) % nby) * kEditY,
@@ -242,7 +269,7 @@ __global__ void __launch_bounds__(NT) k_edit_box(GridDesc g, GridDesc r, FieldWo
         fix |= mine[j] && old[j] < 0 && (sr < 0 || dist2(x, y, z) < sr * sr);
     }
     const bool any = __syncthreads_or(fix) != 0;
-    if (any) dev::field_tile<kEditY, kEditZ, NT>(L, tid, words);
+    if (any) dev::field_tile<kEditY, kEditZ, NT>(L, L.plane, tid);
 #pragma unroll
     for (int j = 0; j < kCells; j++) {
         if (!mine[j]) continue;
@@ -252,7 +279,7 @@ __global__ void __launch_bounds__(NT) k_edit_box(GridDesc g, GridDesc r, FieldWo
         if (any && now < 0 && (sr < 0 || dist2(x, y, z) < sr * sr)) {
             const uint32_t* p = L.plane + row * 6;
             const uint32_t pl[5] = {p[0], p[1], p[2], p[3], p[4]};
-            if (!(p[5] >> (tid & 31) & 1u)) now = L.word[dev::level_at(pl, tid & 31)];
+            if (!(p[5] >> (tid & 31) & 1u)) now = word[dev::level_at(pl, tid & 31)];
         }
         if (now != was[j]) g.vox[(uint64_t)x + g.X * (uint64_t)y + g.XY * (uint64_t)z] = now;
         if (r.vox) r.vox[r.origin + (uint64_t)x + (uint64_t)r.SX * (uint64_t)y + r.SXY * (uint64_t)z] = now;
@@ -306,6 +333,76 @@ __global__ void __launch_bounds__(256) k_solid_top(GridDesc g, int32_t x0, int32
         if (__builtin_amdgcn_ballot_w64(any) != 0) best = y;
     }
     if (lane == 0 && best >= 0) atomicMax(top, best);
+}
+
+// The whole grid in one pass: words from `src` (the grid itself, or a level
+// elsewhere on the device) into the render copy and, when they come from
+// elsewhere, the grid; *top is raised to the highest y of a solid voxel.  A
+// lane moves four voxels of each of kLoadRows rows, all loads in flight
+// together; a block raises *top only when it holds something higher than it
+// already says (one atomic per wave on that word took 0.33 ms by itself).
+// Memory bound: 1 GiB in 0.62 ms (3.2 GB, 5.2 TB/s), against 1.20 ms for three
+// passes (copy 0.49, solid top 0.33, render copy 0.38).
+constexpr int kLoadRows = 4;
+__global__ void __launch_bounds__(256) k_load_grid(GridDesc g, GridDesc r, const int32_t* src, uint64_t rows,
+                                                   uint32_t Q, uint64_t blocks) {
+    __shared__ int32_t best;
+    int32_t high = -1;
+    for (uint64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
+        // quads of four voxels, Q per row; row (y, z) is y + Y * z
+        const uint64_t base = b * 256, rg0 = base / Q;
+        const uint32_t q0 = (uint32_t)(base % Q) + threadIdx.x;
+        const uint64_t row0 = (rg0 + q0 / Q) * kLoadRows;
+        const uint32_t x = q0 % Q * 4;
+        const uint64_t zb = rg0 * kLoadRows / g.Y;
+        uint32_t y = (uint32_t)(rg0 * kLoadRows - zb * g.Y) + q0 / Q * kLoadRows;
+        uint64_t z = zb + y / g.Y;
+        y %= g.Y;
+        const uint32_t n = x + 4 <= g.X ? 4 : g.X - x;
+        dev::vox4 v[kLoadRows];
+#pragma unroll
+        for (int j = 0; j < kLoadRows; j++) {
+            const int32_t* p = src + (row0 + j) * g.X + x;
+            v[j] = -1;
+            if (row0 + j >= rows) continue;
+            if (n == 4) {
+                v[j] = *(const dev::vox4*)p;
+            } else {
+                v[j].x = p[0];
+                if (n > 1) v[j].y = p[1];
+                if (n > 2) v[j].z = p[2];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kLoadRows; j++) {
+            if (row0 + j < rows) {
+                int32_t* c = r.vox + (r.origin + x + (uint64_t)r.SX * y + r.SXY * z);
+                int32_t* d = g.vox + (row0 + j) * g.X + x;
+                if (n == 4) {
+                    *(dev::vox4*)c = v[j];
+                    if (src != g.vox) *(dev::vox4*)d = v[j];
+                } else {
+                    for (uint32_t k = 0; k < n; k++) {
+                        const int32_t w = k == 0 ? v[j].x : (k == 1 ? v[j].y : v[j].z);
+                        c[k] = w;
+                        if (src != g.vox) d[k] = w;
+                    }
+                }
+                if ((v[j].x & v[j].y & v[j].z & v[j].w) >= 0) high = max(high, (int32_t)y);
+            }
+            if (++y == g.Y) {
+                y = 0;
+                z++;
+            }
+        }
+    }
+    if (threadIdx.x == 0) best = __atomic_load_n(g.top, __ATOMIC_RELAXED);
+    __syncthreads();
+    const int32_t seen = best;
+    __syncthreads();
+    if (high > seen) atomicMax(&best, high);
+    __syncthreads();
+    if (threadIdx.x == 0 && best > seen) atomicMax(g.top, best);
 }
 
 // Grid copy, 16 bytes per lane per step (a plain streaming copy of known size).
@@ -392,14 +489,14 @@ int launch_build_depth_field(const GridDesc& g, const GridDesc& render, const Fi
     const uint32_t W = solid_bits_words(g);
     const uint64_t rows = (uint64_t)g.Y * g.Z;
     const uint64_t bit_blocks = ((rows + kBitRows - 1) / kBitRows * (W * 8ull) + 255) / 256;
-    const uint64_t nx = (g.X + 31ull) / 32, ny = (g.Y + kTileY - 1ull) / kTileY, nz = (g.Z + kTileZ - 1ull) / kTileZ;
-    const uint64_t tiles = nx * ny * nz;
-    if (bit_blocks > 0x7fffffffull || nx * ny > 0x7ffffff0ull || tiles > 0x7ffffff0ull)
+    const uint64_t runs = (g.X + 32ull * kTileRun - 1) / (32 * kTileRun), ny = (g.Y + kTileY - 1ull) / kTileY, nz = (g.Z + kTileZ - 1ull) / kTileZ;
+    const uint64_t total = runs * ny * nz;
+    if (bit_blocks > 0x7fffffffull || runs * ny > 0x7ffffff0ull || total > 0x7ffffff0ull)
         return fail(VRT_ERR_INVALID, "grid too large for the build");
     hipLaunchKernelGGL(k_solid_bits, dim3((uint32_t)bit_blocks), dim3(256), 0, s, g, bits, W, rows);
     VRT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_field_tiles, dim3((uint32_t)((tiles + 7) / 8 * 8)), dim3(kTileThreads), 0, s, g, render, words,
-                       bits, W, (uint32_t)nx, (uint32_t)ny, (uint32_t)tiles);
+    hipLaunchKernelGGL(k_field_tiles, dim3((uint32_t)((total + 7) / 8 * 8)), dim3(kTileThreads), 0, s, g, render, words,
+                       bits, W, (uint32_t)runs, (uint32_t)ny, (uint32_t)total);
     VRT_HIP(hipGetLastError());
     return VRT_OK;
 }
@@ -416,6 +513,20 @@ int launch_set_voxel(const GridDesc& g, const GridDesc& render, int32_t x, int32
     return VRT_OK;
 }
 
+int launch_load_grid(const GridDesc& g, const GridDesc& render, const int32_t* src, hipStream_t s) {
+    if (!g.top) return fail(VRT_ERR_INVALID, "grid without a solid-top word");
+    if ((uintptr_t)src & 15) return fail(VRT_ERR_INVALID, "copy buffers must be 16-byte aligned");
+    const uint64_t rows = (uint64_t)g.Y * g.Z;
+    const uint32_t Q = (g.X + 3u) / 4u;
+    const uint64_t blocks = ((rows + kLoadRows - 1) / kLoadRows * Q + 255) / 256;
+    hipLaunchKernelGGL(k_set_word, dim3(1), dim3(64), 0, s, g.top, -1);
+    VRT_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_load_grid, dim3((uint32_t)std::min<uint64_t>(blocks, 1u << 23)), dim3(256), 0, s, g, render,
+                       src, rows, Q, blocks);
+    VRT_HIP(hipGetLastError());
+    return VRT_OK;
+}
+
 int launch_put_box(const GridDesc& g, const GridDesc& render, const int32_t* src, int64_t first, int64_t n, int64_t nx,
                    int64_t ny, int64_t x0, int64_t y0, int64_t z0, int32_t top, hipStream_t s) {
     if (n <= 0) return VRT_OK;
@@ -427,12 +538,8 @@ int launch_put_box(const GridDesc& g, const GridDesc& render, const int32_t* src
 }
 
 int launch_solid_top(const GridDesc& g, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1,
-                     bool reset, hipStream_t s) {
+                     hipStream_t s) {
     if (!g.top) return fail(VRT_ERR_INVALID, "grid without a solid-top word");
-    if (reset) {
-        hipLaunchKernelGGL(k_set_word, dim3(1), dim3(64), 0, s, g.top, -1);
-        VRT_HIP(hipGetLastError());
-    }
     clip(x0, x1, g.X);
     clip(y0, y1, g.Y);
     clip(z0, z1, g.Z);

@@ -101,7 +101,6 @@ struct FieldTile {
         };
         uint32_t plane[kRows * 6];
     };
-    int32_t word[kFieldLevels + 2];
 };
 
 __device__ __forceinline__ uint32_t funnel(uint32_t hi, uint32_t lo, uint32_t shift) {
@@ -113,15 +112,15 @@ __device__ __forceinline__ uint4 or4(uint4 a, uint4 b) {
 }
 
 // From the solidity rows in L.s (written by the caller, before a barrier) to
-// the tile's result in L.plane: for row r = z * TY + y, words 0-4 are bit
-// planes of each voxel's level (0: keep the word, k: L.word[k]) and word 5
-// the voxels whose word is kept (solid, or n < 4).  Every one of the NT
-// threads calls it; it ends on a barrier.
+// the tile's result in `plane` (LDS; L.plane or elsewhere): for row
+// r = z * TY + y, words 6 r to 6 r + 4 are bit planes of each voxel's level
+// (0: keep the word, k: FieldWords::word[k]) and word 6 r + 5 the voxels whose
+// word is kept (solid, or n < 4).  Every one of the NT threads calls it; it
+// ends on a barrier.
 template <int TY, int TZ, int NT>
-__device__ __forceinline__ void field_tile(FieldTile<TY, TZ>& L, int tid, const FieldWords& words) {
+__device__ __forceinline__ void field_tile(FieldTile<TY, TZ>& L, uint32_t* plane, int tid) {
     using T = FieldTile<TY, TZ>;
-    static_assert(NT >= T::kRows && NT >= kFieldLevels + 2, "one thread per row of the tile");
-    if (tid < kFieldLevels + 2) L.word[tid] = words.word[tid];
+    static_assert(NT >= T::kRows, "one thread per row of the tile");
     // D: dilate along y, then z, then x; the masks X_a of each row
     for (int i = tid; i < T::SZ * T::DY; i += NT) {
         const int r = (i / T::DY) * T::SY + i % T::DY;
@@ -214,7 +213,7 @@ __device__ __forceinline__ void field_tile(FieldTile<TY, TZ>& L, int tid, const 
 #pragma unroll
         for (int k = 3; k <= kFieldLevels; k += 4) p2 ^= t[k];
         static_assert(kFieldLevels == 23, "24 flags: even counts for planes 0-2, three for plane 3, one for plane 4");
-        uint32_t* p = L.plane + tid * 6;
+        uint32_t* p = plane + tid * 6;
         p[0] = p0;
         p[1] = p1;
         p[2] = p2;

@@ -172,15 +172,18 @@ int launch_build_depth_field(const GridDesc& g, const GridDesc& render, const Fi
 // One voxel of the grid and of the render copy; raises *g.top for a solid one.
 int launch_set_voxel(const GridDesc& g, const GridDesc& render, int32_t x, int32_t y, int32_t z, int32_t v,
                      hipStream_t s);
+// The whole grid from `src` (device; g.vox: the grid itself) into the render
+// copy and the grid; sets *g.top to the highest y with a solid voxel.
+int launch_load_grid(const GridDesc& g, const GridDesc& render, const int32_t* src, hipStream_t s);
 // Words [first, first + n) of the box at (x0, y0, z0), nx x ny voxels per z,
 // from pinned host memory into the grid and the render copy; raises *g.top to
 // `top`.
 int launch_put_box(const GridDesc& g, const GridDesc& render, const int32_t* src, int64_t first, int64_t n, int64_t nx,
                    int64_t ny, int64_t x0, int64_t y0, int64_t z0, int32_t top, hipStream_t s);
 // Raises *g.top to the highest y with a solid voxel in the box [x0,x1) x
-// [y0,y1) x [z0,z1) (clipped to the grid); with reset, sets it to -1 first.
+// [y0,y1) x [z0,z1) (clipped to the grid).
 int launch_solid_top(const GridDesc& g, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1,
-                     bool reset, hipStream_t s);
+                     hipStream_t s);
 int launch_fill(int32_t* p, uint64_t n, int32_t v, hipStream_t s);
 // dst's cells of the box [x0,x0+nx) x [y0,y0+ny) x [z0,z0+nz) := src's.
 int launch_copy_box(const GridDesc& src, const GridDesc& dst, int64_t x0, int64_t y0, int64_t z0, int64_t nx,
@@ -244,11 +247,9 @@ inline GridDesc render_grid(const vrt_ctx* c) {
     g.top = c->shadow_cutoff ? c->grid.top : nullptr;
     return g;
 }
-int solid_top_full(vrt_ctx* c);  // recomputes *grid.top over the whole grid
 // Copies the box [x0,x1) x [y0,y1) x [z0,z1) (clipped to the grid) of the
 // grid into the render copy, on the context's stream.
 int refresh_render(vrt_ctx* c, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1);
-int refresh_render_all(vrt_ctx* c);
 // removeSphere on stream s: carve and depth-field repair of the grid and, unless
 // render.vox is null, of the edited box of that padded copy.
 int remove_sphere_on(vrt_ctx* c, const GridDesc& render, int32_t cx, int32_t cy, int32_t cz, int32_t radius,
