@@ -1,0 +1,86 @@
+"""The written-out walk (vrt_device.h: cast_ray, run_walk) where its arithmetic
+differs in form from the shader's: whole coordinates after a jump, ties, walks
+that leave the grid by a low face or by the x-y edge, starts outside its range.
+Against the oracle's castRay, bit for bit, for 32-bit byte offsets and 32-bit
+indices."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [(24, 20, 40), (4096, 600, 2)]  # byte offsets; 4 X Y >= 2^23: word indices
+
+
+def compare(gpu, orc, world, dims, start, d, dist, budget=256):
+    start, d = np.asarray(start, np.float32), np.asarray(d, np.float32)
+    dist = np.asarray(dist, np.int32)
+    ctx = gpu.Context(dims)
+    ctx.upload(world)
+    r = orc.cast_rays(world, dims, start, d, dist, budget)
+    for steps in (True, False):
+        g = ctx.cast_rays(start, d, dist, budget, steps=steps)
+        for k in ("hit", "face", "steps") if steps else ("hit", "face"):
+            bad = np.nonzero(g[k] != r[k])[0]
+            assert bad.size == 0, "%s differs for %d rays, first start %s dir %s: %s, oracle %s" % (
+                k, bad.size, start[bad[0]].tolist(), d[bad[0]].tolist(), g[k][bad[0]], r[k][bad[0]])
+        # bitwise, any NaN equal to any NaN
+        same = (g["hit_pos"].view(np.uint32) == r["hit_pos"].view(np.uint32)) | (np.isnan(g["hit_pos"]) & np.isnan(r["hit_pos"]))
+        bad = np.nonzero(~same.all(1))[0]
+        assert bad.size == 0, "hit_pos differs for %d rays, first start %s dir %s: %s, oracle %s" % (
+            bad.size, start[bad[0]].tolist(), d[bad[0]].tolist(), g["hit_pos"][bad[0]], r["hit_pos"][bad[0]])
+    ctx.close()
+    return r
+
+
+@pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_walks_on_dyadic_numbers(gpu, orc, dims, seed):
+    """Starts, directions and jumps that are small multiples of powers of two:
+    every product and sum is exact, so coordinates after a jump are often whole
+    and intersects often equal."""
+    rng = np.random.default_rng(seed)
+    X, Y, Z = dims
+    cells = X * Y * Z
+    world = np.full(cells, -1, np.int32)
+    jump = rng.random(cells) < 0.5
+    world[jump] = (-0.5 * rng.integers(1, 17, int(jump.sum())).astype(np.float32)).view(np.int32)
+    solid = rng.random(cells) < 0.04
+    world[solid] = rng.integers(0, 1 << 24, int(solid.sum()))
+    n = 40000
+    start = np.stack([rng.integers(0, 4 * min(s, 48), n) / 4.0 for s in dims], 1)
+    start += rng.choice([0.0, 0.0, 0.5, 2.0 ** -20, 2.0 ** -21], (n, 1))
+    far = rng.random(n) < 0.3  # near the high faces
+    start[far] = np.array(dims) - start[far]
+    d = rng.choice([-1.0, -0.5, -0.25, 0.25, 0.5, 1.0], (n, 3))
+    some = rng.random(n) < 0.1
+    d[some, rng.integers(0, 3)] = 0.0
+    r = compare(gpu, orc, world, dims, start, d, rng.integers(1, 200, n))
+    assert int((r["hit"] >= 0).sum()) > 1000  # 5-6% of the rays on the flat grid
+
+
+def test_leaving_by_the_edge_with_equal_intersects(gpu, orc):
+    """A jump that leaves x and y in (-1, 0), both heading down, with equal
+    (negative) intersects: the shader steps z and stays in the cell column
+    x = y = 0 until a solid voxel, a jump or the grid's end."""
+    dims = (12, 12, 40)
+    X, Y, _ = dims
+    starts, dirs, worlds = [], [], []
+    for dz in (0.3, -0.3):
+        for zs in (1, 2, 5):  # z steps from the jump's end to the solid voxel
+            z0 = 5.5 if dz > 0 else 30.5
+            w = np.full(dims[0] * dims[1] * dims[2], -1, np.int32)
+            first = 6 if dz > 0 else 29  # x and y tie at the start too: z is stepped
+            w[2 + X * 2 + X * Y * first] = np.float32(-(6.0 - 0.5 / 0.3)).view(np.int32)
+            end = int(z0 + dz * 6.0)
+            w[X * Y * (end + (zs if dz > 0 else -zs))] = 0x112233
+            starts.append([2.5, 2.5, z0])
+            dirs.append([-0.5, -0.5, dz])
+            worlds.append(w)
+    hits = 0
+    for s, d, w in zip(starts, dirs, worlds):
+        n = 70  # more than one wave, the other lanes on other walks
+        start = np.repeat(np.array([s]), n, 0)
+        start[1::2, 0] += np.linspace(0.1, 3.0, n)[1::2]
+        r = compare(gpu, orc, w, dims, start, np.repeat(np.array([d]), n, 0), np.full(n, 200))
+        hits += int((r["hit"][::2] >= 0).sum())
+    assert hits == 6 * 35, hits  # every such ray reaches its voxel

@@ -397,7 +397,7 @@ int vrt_create(vrt_ctx** out, int64_t X, int64_t Y, int64_t Z, int32_t device) {
     if ((e = hipMemsetAsync(c->counters, 0, counter_bytes, c->stream)) != hipSuccess)
         return bail(hip_fail(e, "hipMemsetAsync"));
     rc = launch_fill(c->grid.vox, count, -1, c->stream);
-    if (!rc) rc = launch_fill(c->rgrid.vox, c->rgrid.count, kGuardValue, c->stream);
+    if (!rc) rc = launch_fill_guard(c->rgrid, c->stream);
     if (!rc) rc = launch_load_grid(c->grid, c->rgrid, c->grid.vox, c->stream);
     if (rc) return bail(rc);
     c->top_host = -1;

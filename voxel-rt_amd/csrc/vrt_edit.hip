@@ -444,6 +444,11 @@ __global__ void __launch_bounds__(256) k_fill(int32_t* p, uint64_t n, int32_t v)
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
 
+__global__ void __launch_bounds__(64) k_fill_corner(GridDesc r) {
+    const uint32_t i = threadIdx.x, z = blockIdx.x;
+    if (i < kGuard * kGuard) r.vox[i % kGuard + (uint64_t)r.SX * (i / kGuard) + r.SXY * z] = kGuardCorner;
+}
+
 // Clip [lo, hi) to [0, n).
 inline void clip(int64_t& lo, int64_t& hi, int64_t n) {
     if (lo < 0) lo = 0;
@@ -585,6 +590,13 @@ int launch_fill(int32_t* p, uint64_t n, int32_t v, hipStream_t s) {
     uint64_t blocks = (n + 255) / 256;
     if (blocks > 65536ull * 16) blocks = 65536ull * 16;
     hipLaunchKernelGGL(k_fill, dim3((uint32_t)blocks), dim3(256), 0, s, p, n, v);
+    VRT_HIP(hipGetLastError());
+    return VRT_OK;
+}
+
+int launch_fill_guard(const GridDesc& render, hipStream_t s) {
+    if (int rc = launch_fill(render.vox, render.count, kGuardValue, s)) return rc;
+    hipLaunchKernelGGL(k_fill_corner, dim3((uint32_t)(render.Z + 2 * kGuard)), dim3(64), 0, s, render);
     VRT_HIP(hipGetLastError());
     return VRT_OK;
 }

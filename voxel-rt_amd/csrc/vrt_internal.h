@@ -29,6 +29,9 @@ int hip_fail(hipError_t e, const char* what);
 // walk the same way in the reference, :114-121 then :83.)
 constexpr int32_t kGuard = 3;
 constexpr int32_t kGuardValue = (int32_t)0xFFC00000u;
+// The guard cells with x < 0 and y < 0 hold another NaN, by which a walk knows
+// that it left the grid there (cast_ray).
+constexpr int32_t kGuardCorner = (int32_t)0xFFC00001u;
 
 // Grid as the kernels see it.  Cell (x, y, z) is vox[origin + x + SX*y +
 // SXY*z]; X, Y, Z are the grid's extents.  The library's grid is dense
@@ -185,6 +188,8 @@ int launch_put_box(const GridDesc& g, const GridDesc& render, const int32_t* src
 int launch_solid_top(const GridDesc& g, int64_t x0, int64_t y0, int64_t z0, int64_t x1, int64_t y1, int64_t z1,
                      hipStream_t s);
 int launch_fill(int32_t* p, uint64_t n, int32_t v, hipStream_t s);
+// Every word of a padded copy: kGuardCorner where x < 0 and y < 0, else kGuardValue.
+int launch_fill_guard(const GridDesc& render, hipStream_t s);
 // dst's cells of the box [x0,x0+nx) x [y0,y0+ny) x [z0,z0+nz) := src's.
 int launch_copy_box(const GridDesc& src, const GridDesc& dst, int64_t x0, int64_t y0, int64_t z0, int64_t nx,
                     int64_t ny, int64_t nz, hipStream_t s);

@@ -99,11 +99,7 @@ k_render_plain(GridDesc g, FrameDesc F, vrt_target t, unsigned long long* counte
         if (px < t.width && row < t.height) {
             float vx, vy;
             dev::pixel_vpos(t.width, t.height, F.inv_w, F.inv_h, px, row, vx, vy);
-            dev::PixelResult p;
-            dev::shade_pixel<IX>(g, F, vx, vy, p, top);
-            dev::store_pixel<IX>(g, t, (int64_t)row * t.width + px, p);
-            rays = p.rays;
-            iters = p.iters;
+            dev::shade_pixel<IX>(g, F, t, (int64_t)row * t.width + px, vx, vy, top, rays, iters);
             pixels = 1;
         }
     }
@@ -140,8 +136,8 @@ __global__ void __launch_bounds__(256) k_cast_rays(GridDesc g, int64_t n, const 
     // the cutoff applies when the caller does not ask for the step counts
     const float dy = dir[3 * i + 1];
     dev::Hit h;
-    dev::cast_ray<IX>(g, start[3 * i], start[3 * i + 1], start[3 * i + 2], dir[3 * i], dy, dir[3 * i + 2], lim, h,
-                      (steps == nullptr && dy >= 0.0f) ? top : INT32_MAX);
+    dev::cast_ray<IX, false>(g, start[3 * i], start[3 * i + 1], start[3 * i + 2], dir[3 * i], dy, dir[3 * i + 2], lim, h,
+                      steps == nullptr ? top : INT32_MAX);
     const bool hitp = h.index != -1;
     if (hit) hit[i] = hitp ? IX::ref_index(g, h.index) : -1;
     if (hit_pos) {
@@ -187,11 +183,10 @@ __device__ __forceinline__ void shade_view_tile(const GridDesc& g, const ViewDes
         if (px < V.target.width && row < V.target.height) {
             float vx, vy;
             dev::pixel_vpos(V.target.width, V.target.height, V.frame.inv_w, V.frame.inv_h, px, row, vx, vy);
-            dev::PixelResult p;
-            dev::shade_pixel<IX>(g, V.frame, vx, vy, p, top);
-            dev::store_pixel<IX>(g, V.target, (int64_t)row * V.target.width + px, p);
-            rays += p.rays;
-            iters += p.iters;
+            uint32_t r, n;
+            dev::shade_pixel<IX>(g, V.frame, V.target, (int64_t)row * V.target.width + px, vx, vy, top, r, n);
+            rays += r;
+            iters += n;
             pixels += 1;
         }
     }
