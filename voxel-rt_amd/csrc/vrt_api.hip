@@ -111,8 +111,10 @@ FrameDesc make_frame_desc(const vrt_frame& f, const vrt_target& target) {
     d.inv_h = height > 0 ? 1.0f / (float)height : 0.0f;
     d.primary_cutoff = (f.view_depth_field != 1 && target.steps == nullptr) ? 1 : 0;
     d.row_rot = 0;
+    d.tiles_rcp = tile_rcp((uint32_t)(width + 7) / 8);  // the plain draw's 8x8 tiles; make_view_desc sets its own
     for (int i = 0; i < VRT_MAX_LOCAL_LIGHTS; i++) {
         const vrt_local_light& L = f.lights[i];
+        d.light_x[i] = L.pos[0];
         d.light_dd_max[i] = sqrt_le_limit(L.radius);
         d.light_axis_max[i] = square_le_limit(d.light_dd_max[i]);
         d.light_rinv[i] = 1.0f / L.radius;
@@ -379,6 +381,9 @@ int vrt_create(vrt_ctx** out, int64_t X, int64_t Y, int64_t Z, int32_t device) {
         r.SXY = PX * PY;
         r.count = PX * PY * PZ;
         r.origin = (uint64_t)kGuard * (1 + PX + PX * PY);
+        r.FX = (float)std::min<int64_t>(X, 1 << 22);
+        r.FY = (float)std::min<int64_t>(Y, 1 << 22);
+        r.FZ = (float)std::min<int64_t>(Z, 1 << 22);
         r.vox = nullptr;
         if (hipMalloc(&r.vox, r.count * sizeof(int32_t)) != hipSuccess) {
             (void)hipGetLastError();

@@ -76,6 +76,7 @@ int make_view_desc(const vrt_view& v, const vrt_batch_config& cfg, int64_t first
     d.frame = make_frame_desc(v.frame, v.target);
     d.target = v.target;
     d.tiles_x = (v.target.width + cfg.tile_w - 1) / cfg.tile_w;
+    d.frame.tiles_rcp = tile_rcp((uint32_t)d.tiles_x);
     const int32_t tiles_y = (v.target.height + cfg.tile_h - 1) / cfg.tile_h;
     d.tiles = d.tiles_x * tiles_y;
     d.first_tile = first_tile;

@@ -29,6 +29,13 @@ __device__ __forceinline__ int32_t f2i(float v) {
     return r;
 }
 
+// Largest integer not above v.
+__device__ __forceinline__ int32_t floor_i(float v) {
+    int32_t r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+
 // int(sign(v)) (src/fshader.glsl:71); sign(NaN) = 0.
 __device__ __forceinline__ int32_t isign(float v) { return v > 0.0f ? 1 : (v < 0.0f ? -1 : 0); }
 
@@ -122,6 +129,7 @@ struct Hit {
     float pos[3];    // hitPos (valid on a hit)
     int32_t axis;    // axis of the step into the hit voxel (-1 on a miss)
     int32_t step;    // step on that axis
+    int32_t word;    // the hit voxel's word
     uint32_t iters;  // loop iterations (stepCount increments)
 };
 
@@ -169,6 +177,11 @@ struct IdxB {
     __device__ __forceinline__ static int32_t load(const int32_t* vox, T i) {
         return *(const int32_t*)((const char*)vox + i);
     }
+    // i + c * stride, both factors within signed 24 bits
+    __device__ __forceinline__ static T add(T i, int32_t c, int32_t stride) {
+        asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(i) : "v"(c), "v"(stride), "v"(i));
+        return i;
+    }
     __device__ __forceinline__ static int64_t word(T i) { return (int64_t)(i >> 2); }
     __device__ __forceinline__ static int64_t ref_index(const GridDesc& g, int64_t w) {
         return ref_index_of<uint32_t>(g, (uint32_t)w - (uint32_t)g.origin);
@@ -186,6 +199,11 @@ struct Idx32 {
         return (uint32_t)step * (axis == 0 ? 1u : (axis == 1 ? g.SX : (uint32_t)g.SXY));
     }
     __device__ __forceinline__ static int32_t load(const int32_t* vox, T i) { return vox[i]; }
+    // i + c * stride, both factors within signed 24 bits
+    __device__ __forceinline__ static T add(T i, int32_t c, int32_t stride) {
+        asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(i) : "v"(c), "v"(stride), "v"(i));
+        return i;
+    }
     __device__ __forceinline__ static int64_t word(T i) { return (int64_t)i; }
     __device__ __forceinline__ static int64_t ref_index(const GridDesc& g, int64_t w) {
         return ref_index_of<uint32_t>(g, (uint32_t)w - (uint32_t)g.origin);
@@ -291,6 +309,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
             h.pos[2] = dz * cur + sz;
             axis = bx ? 0 : (by ? 1 : 2);
             result = IX::word(idx);
+            h.word = v;
             break;
         }
         if (v != -1) {
@@ -358,9 +377,8 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // word index is base + sum of floor(s') times the step's negated stride; base
 // takes up the 1.
 //
-// Which rays: those whose direction components and the sums d + 1e-6 lie in
-// [2^-60, 2^60] in magnitude and whose start coordinates lie in [2^-20, 2^22]
-// (cast_ray).  On an ascending axis s then stays at least 2^-20, where the
+// Which rays: those whose direction components lie in [2^-19, 2^60] in
+// magnitude and whose start coordinates lie in [2^-20, 2^22] (cast_ray).  On an ascending axis s then stays at least 2^-20, where the
 // hardware's fraction is the rounded difference; on a descending one s may
 // fall below 0 only on its way out of the grid (below).  Only the low end of a
 // cell is clamped (lo: clamp_cell's -2 or n + 1, mirrored): a ray jumps from
@@ -575,43 +593,52 @@ __device__ __forceinline__ void run_walk(Idx32, const int32_t* vox, float lim, u
 #undef VRT_WALK_IN
 
 // castRay, src/fshader.glsl:59-129 (see walk_generic for lim), from p, or with
-// kOffset from p + d * 0.001 (the shadow rays' start, :152, :165).  ytop: the
-// cutoff's bound for a ray that does not head down (INT32_MAX: none).  What the
+// kHit from p + d * 0.001 (the shadow rays' start, :152, :165).  ytop: the cutoff's
+// bound for a ray that does not head down (INT32_MAX: none).  What the
 // walk does not need is recovered from its state afterwards (the direction and
 // steps from d' and the strides, the start from p) rather than held in
 // registers meanwhile.
-template <typename IX, bool kOffset>
+//
+// The first cell and intersects.  From a hit: as after a jump, for a start
+// inside the grid (any other takes walk_generic).  Else: the reference's
+// formulas.  (The camera's distances to its cell's boundaries made with the
+// frame instead of by every lane: no gain, small frames 2% slower.)
+template <typename IX, bool kHit>
 __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, float pz, float dx, float dy,
                                          float dz, float lim, Hit& h, int32_t ytop) {
     bool general = true;
     if constexpr (!std::is_same_v<IX, Idx64>) {
-        const float sx = kOffset ? px + dx * 0.001f : px, sy = kOffset ? py + dy * 0.001f : py,
-                    sz = kOffset ? pz + dz * 0.001f : pz;
-        const float bx_ = fabsf(dx + 0.000001f), by_ = fabsf(dy + 0.000001f), bz_ = fabsf(dz + 0.000001f);
-        const float lo = fminf(fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz)), fminf(fminf(bx_, by_), bz_));
-        const float hi = fmaxf(fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz)), fmaxf(fmaxf(bx_, by_), bz_));
-        const bool dok = (lo >= 0x1p-60f) & (hi <= 0x1p60f);
-        const float sum = ((dx + dy) + dz) + ((sx + sy) + sz);  // a NaN among them, which min and max pass over
-        if (dok && fminf(fminf(sx, sy), sz) >= 0x1p-20f && fmaxf(fmaxf(sx, sy), sz) <= 0x1p22f && sum == sum) {
-            Walk w;
-            const bool mx = dx > 0.0f, my = dy > 0.0f, mz = dz > 0.0f;
-            const int32_t cx = f2i(sx), cy = f2i(sy), cz = f2i(sz);
-            w.ddx = rcp_fast(bx_);
-            w.ddy = rcp_fast(by_);
-            w.ddz = rcp_fast(bz_);
+        const float sx = kHit ? px + dx * 0.001f : px, sy = kHit ? py + dy * 0.001f : py,
+                    sz = kHit ? pz + dz * 0.001f : pz;
+        Walk w;
+        const bool mx = dx > 0.0f, my = dy > 0.0f, mz = dz > 0.0f;
+        w.sx = mx ? -sx : sx;
+        w.sy = my ? -sy : sy;
+        w.sz = mz ? -sz : sz;
+        // |d| >= 2^-19 keeps |d + 1e-6| in range too.  min and max pass over a
+        // NaN; the comparisons of s (NaN where d is) or the sum do not.
+        const float lo = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
+        const float hi = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz));
+        bool fast = (lo >= 0x1p-19f) & (hi <= 0x1p60f);
+        if constexpr (kHit) {
+            w.ix = __builtin_amdgcn_fractf(w.sx);
+            w.iy = __builtin_amdgcn_fractf(w.sy);
+            w.iz = __builtin_amdgcn_fractf(w.sz);
+            fast &= (fminf(fminf(sx, sy), sz) >= 0x1p-20f) & (sx < g.FX) & (sy < g.FY) & (sz < g.FZ);
+        } else {
+            const float sum = ((dx + dy) + dz) + ((sx + sy) + sz);
+            fast &= (fminf(fminf(sx, sy), sz) >= 0x1p-20f) & (fmaxf(fmaxf(sx, sy), sz) <= 0x1p22f) & (sum == sum);
+        }
+        if (fast) {
+            w.ddx = rcp_fast(fabsf(dx + 0.000001f));
+            w.ddy = rcp_fast(fabsf(dy + 0.000001f));
+            w.ddz = rcp_fast(fabsf(dz + 0.000001f));
             w.rx = rcp_fast(fabsf(dx));
             w.ry = rcp_fast(fabsf(dy));
             w.rz = rcp_fast(fabsf(dz));
             w.dx = -fabsf(dx);
             w.dy = -fabsf(dy);
             w.dz = -fabsf(dz);
-            w.sx = mx ? -sx : sx;
-            w.sy = my ? -sy : sy;
-            w.sz = mz ? -sz : sz;
-            // the quotients (c + f - s) / d, numerators mirrored too
-            div3_by((float)(mx ? -cx - 1 : cx) - w.sx, (float)(my ? -cy - 1 : cy) - w.sy,
-                    (float)(mz ? -cz - 1 : cz) - w.sz, w.dx, w.dy, w.dz, -w.rx, -w.ry, -w.rz, true, w.ix, w.iy, w.iz);
-            w.idx = IX::make(g, clamp_cell(cx, g.X), clamp_cell(cy, g.Y), clamp_cell(cz, g.Z));
             w.nstx = (int32_t)IX::stride(g, mx ? -1 : 1, 0);
             w.nsty = (int32_t)IX::stride(g, my ? -1 : 1, 1);
             w.nstz = (int32_t)IX::stride(g, mz ? -1 : 1, 2);
@@ -619,6 +646,36 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
             w.loy = my ? -(int32_t)g.Y - 2 : -2;
             w.loz = mz ? -(int32_t)g.Z - 2 : -2;
             w.base = IX::make(g, 0, 0, 0) + (uint32_t)((mx ? w.nstx : 0) + (my ? w.nsty : 0) + (mz ? w.nstz : 0));
+            if constexpr (kHit) {
+                // u / |d| as after a jump: exact for u = 0 and u >= 2^-60
+                auto quotient = [](float u, float d, float r) {
+                    const float q0 = u * r;
+                    return __builtin_fmaf(__builtin_fmaf(q0, d, u), r, q0);
+                };
+                w.idx = IX::add(w.base, floor_i(w.sx), w.nstx);
+                w.idx = IX::add(w.idx, floor_i(w.sy), w.nsty);
+                w.idx = IX::add(w.idx, floor_i(w.sz), w.nstz);
+                // s >= 2^-20, so a fraction is 0 or at least 2^-43.  A whole s
+                // on an ascending axis: the boundary ahead is 1 away, the
+                // cell one lower than floor(s') says.  (Common: a face's
+                // coordinate stays whole where d * 0.001 rounds away.)
+                if (fminf(fminf(w.ix, w.iy), w.iz) == 0.0f) {
+                    const bool ax = mx & (w.ix == 0.0f), ay = my & (w.iy == 0.0f), az = mz & (w.iz == 0.0f);
+                    w.idx -= (uint32_t)((ax ? w.nstx : 0) + (ay ? w.nsty : 0) + (az ? w.nstz : 0));
+                    w.ix = ax ? 1.0f : w.ix;
+                    w.iy = ay ? 1.0f : w.iy;
+                    w.iz = az ? 1.0f : w.iz;
+                }
+                w.ix = quotient(w.ix, w.dx, w.rx);
+                w.iy = quotient(w.iy, w.dy, w.ry);
+                w.iz = quotient(w.iz, w.dz, w.rz);
+            } else {
+                const int32_t cx = f2i(sx), cy = f2i(sy), cz = f2i(sz);
+                w.idx = IX::make(g, clamp_cell(cx, g.X), clamp_cell(cy, g.Y), clamp_cell(cz, g.Z));
+                div3_by((float)(mx ? -cx - 1 : cx) - w.sx, (float)(my ? -cy - 1 : cy) - w.sy,
+                        (float)(mz ? -cz - 1 : cz) - w.sz, w.dx, w.dy, w.dz, -w.rx, -w.ry, -w.rz, true, w.ix, w.iy,
+                        w.iz);
+            }
             w.tb = my ? -1 - ytop : INT32_MIN;
             w.trav = 0.0f;
             w.iters = 0;
@@ -634,6 +691,7 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
             h.axis = hit ? (bx ? 0 : (by ? 1 : 2)) : -1;
             h.step = (bx ? w.nstx : (by ? w.nsty : w.nstz)) < 0 ? 1 : -1;
             h.index = hit ? IX::word(w.idx) : -1;
+            h.word = w.word;
             h.iters = w.iters;
             general = w.word == kGuardCorner;
             dx = flip(w.nstx, w.dx);
@@ -642,8 +700,8 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
         }
     }
     if (__builtin_expect(general, 0))
-        walk_generic<IX>(g, kOffset ? px + dx * 0.001f : px, kOffset ? py + dy * 0.001f : py,
-                         kOffset ? pz + dz * 0.001f : pz, dx, dy, dz, lim, h, dy >= 0.0f ? ytop : INT32_MAX);
+        walk_generic<IX>(g, kHit ? px + dx * 0.001f : px, kHit ? py + dy * 0.001f : py, kHit ? pz + dz * 0.001f : pz,
+                         dx, dy, dz, lim, h, dy >= 0.0f ? ytop : INT32_MAX);
 }
 
 // main(), src/fshader.glsl:131-190, for the fragment at vPos = (vx, vy), pixel
@@ -700,7 +758,7 @@ __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& 
         col1 = s;
         col2 = s;
     } else if (hit) {
-        const int32_t vcol = g.vox[h.index];
+        const int32_t vcol = h.word;
         // toLight = normalize(lightPos - firstHitPos) (:147)
         const float lx0 = f.light_pos[0] - hx, ly0 = f.light_pos[1] - hy, lz0 = f.light_pos[2] - hz;
         const float ln = rcp_rn(sqrtf(dot3(lx0, ly0, lz0, lx0, ly0, lz0)));
@@ -737,15 +795,23 @@ __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& 
             m1 = 1.25f;
             m2 = 1.25f;
         }
-        for (uint32_t rem = F.light_valid; rem != 0u; rem &= rem - 1u) {
+        // The x distance alone rules most lights out for the whole wave: the
+        // lights that it leaves to any lane, four at a time (their x and
+        // bounds lie together, so a group waits for one scalar load; one light
+        // after the other, each waiting for its own, took 3% of a frame with
+        // 16 lights).
+        uint32_t near = 0;
+        for (int j = 0; j < VRT_MAX_LOCAL_LIGHTS && (F.light_valid >> j) != 0u; j += 4) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                near |= __ballot(fabsf(F.light_x[j + i] - hx) <= F.light_axis_max[j + i]) != 0 ? 1u << (j + i) : 0u;
+        }
+        for (uint32_t rem = near & F.light_valid; rem != 0u; rem &= rem - 1u) {
             if (over) break;
             const int i = __builtin_ctz(rem);
             const vrt_local_light& L = f.lights[i];
-            // length <= radius (:171), decided without the square root; the
-            // x distance alone rules most lights out for the whole wave
-            const float vx0 = L.pos[0] - hx;
-            if (!(fabsf(vx0) <= F.light_axis_max[i])) continue;
-            const float vy0 = L.pos[1] - hy, vz0 = L.pos[2] - hz;
+            // length <= radius (:171), decided without the square root
+            const float vx0 = L.pos[0] - hx, vy0 = L.pos[1] - hy, vz0 = L.pos[2] - hz;
             const float dd = dot3(vx0, vy0, vz0, vx0, vy0, vz0);
             if (!(dd <= F.light_dd_max[i])) continue;
             const float dist = sqrtf(dd);

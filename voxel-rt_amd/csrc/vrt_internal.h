@@ -51,6 +51,9 @@ struct GridDesc {
     // kernels stop a shadow ray once it is provably above it; null: they walk
     // every shadow ray to the reference's end.
     int32_t* top;
+    // The extents as floats, at most 2^22 (render copies): a start below them
+    // lies inside the grid and in the range of the walk's arithmetic.
+    float FX, FY, FZ;
     // The y and z a walk can index (the grid's and two cells past it on
     // either side) fit signed 24-bit multiplies.
     bool yz24() const { return (uint64_t)Y + 2 < (1ull << 23) && (uint64_t)Z + 2 < (1ull << 23); }
@@ -61,6 +64,10 @@ struct GridDesc {
         return count <= (1ull << 30) && 4ull * SX < (1ull << 23) && 4ull * SXY < (1ull << 23) && yz24();
     }
 };
+
+// floor(2^32 / d), at most 2^32 - 1: with it a kernel divides by d on the
+// scalar unit.
+inline uint32_t tile_rcp(uint32_t d) { return d <= 1 ? 0xffffffffu : (uint32_t)(((uint64_t)1 << 32) / d); }
 
 // One frame as the kernels see it: vrt_frame plus derived per-frame values.
 struct FrameDesc {
@@ -73,11 +80,13 @@ struct FrameDesc {
     // dot(v, v) >= RN(v.x * v.x) (a sum of non-negative terms, each rounding
     // monotone), so |v.x| > a already puts the light out of range.
     float light_axis_max[VRT_MAX_LOCAL_LIGHTS];
+    float light_x[VRT_MAX_LOCAL_LIGHTS];  // the lights' x
     // Bit i set when light i is placed: every coordinate >= 0 (unused slots
     // hold -1, src/render.cpp:304-311; NaN compares false).
     uint32_t light_valid;
     float light_rinv[VRT_MAX_LOCAL_LIGHTS];  // RN(1 / radius)
     float inv_w, inv_h;                      // RN(1 / width), RN(1 / height) of the target
+    uint32_t tiles_rcp;                      // tile_rcp(tiles across), for the kernels' tile arithmetic
     // Primary rays may stop above every solid voxel too: only when nothing
     // shows their step count (no depth view, no step map in the target).
     int32_t primary_cutoff;

@@ -37,6 +37,17 @@ constexpr int kPlainThreads = kWave * kPlainWaves;
 constexpr int kXcds = 8;
 constexpr int kQueueStride = 32;  // queue counters 128 bytes apart
 
+// n / d and n % d for a wave-uniform n, on the scalar unit, from rcp =
+// tile_rcp(d) (FrameDesc): the product's high word is the quotient or one less.
+__device__ __forceinline__ void split_tile(uint32_t n, uint32_t d, uint32_t rcp, uint32_t& q, uint32_t& r) {
+    q = __umulhi(n, rcp);
+    r = n - q * d;
+    if (r >= d) {
+        r -= d;
+        q++;
+    }
+}
+
 // Adds this wave's totals into its counter slot (see kCounterSlots).
 // Every lane of the wave must be active.  Per-lane totals are 32-bit sums of
 // per-pixel counts, far below 2^58.
@@ -92,9 +103,11 @@ k_render_plain(GridDesc g, FrameDesc F, vrt_target t, unsigned long long* counte
     const int32_t lane = threadIdx.x & 63;
     uint32_t rays = 0, iters = 0, pixels = 0;
     if (tile < tiles_x * tiles_y) {
-        int32_t trow = tile / tiles_x + F.row_rot;
+        uint32_t tq, tr;
+        split_tile((uint32_t)tile, (uint32_t)tiles_x, F.tiles_rcp, tq, tr);
+        int32_t trow = (int32_t)tq + F.row_rot;
         if (trow >= tiles_y) trow -= tiles_y;
-        const int32_t px = (tile % tiles_x) * 8 + (lane & 7);
+        const int32_t px = (int32_t)tr * 8 + (lane & 7);
         const int32_t row = trow * 8 + (lane >> 3);
         if (px < t.width && row < t.height) {
             float vx, vy;
@@ -134,10 +147,9 @@ __global__ void __launch_bounds__(256) k_cast_rays(GridDesc g, int64_t n, const 
     float lim = (float)dist[i];
     lim = lim < render_lim ? lim : render_lim;
     // the cutoff applies when the caller does not ask for the step counts
-    const float dy = dir[3 * i + 1];
     dev::Hit h;
-    dev::cast_ray<IX, false>(g, start[3 * i], start[3 * i + 1], start[3 * i + 2], dir[3 * i], dy, dir[3 * i + 2], lim, h,
-                      steps == nullptr ? top : INT32_MAX);
+    dev::cast_ray<IX, false>(g, start[3 * i], start[3 * i + 1], start[3 * i + 2], dir[3 * i], dir[3 * i + 1],
+                             dir[3 * i + 2], lim, h, steps == nullptr ? top : INT32_MAX);
     const bool hitp = h.index != -1;
     if (hit) hit[i] = hitp ? IX::ref_index(g, h.index) : -1;
     if (hit_pos) {
@@ -174,9 +186,10 @@ __device__ __forceinline__ void shade_view_tile(const GridDesc& g, const ViewDes
         else hi = mid - 1;
     }
     const ViewDesc& V = views[__builtin_amdgcn_readfirstlane(lo)];
-    const int32_t local = (int32_t)(tile - V.first_tile);
-    const int32_t tx0 = (local % V.tiles_x) * TW;
-    const int32_t ty0 = (local / V.tiles_x) * TH;
+    uint32_t tq, tr;
+    split_tile((uint32_t)(tile - V.first_tile), (uint32_t)V.tiles_x, V.frame.tiles_rcp, tq, tr);
+    const int32_t tx0 = (int32_t)tr * TW;
+    const int32_t ty0 = (int32_t)tq * TH;
     const int32_t px = tx0 + (lane & (TW - 1));
     for (int32_t pass = first_pass; pass < first_pass + n_passes; pass++) {
         const int32_t row = ty0 + pass * kRowsPerPass + lane / TW;
