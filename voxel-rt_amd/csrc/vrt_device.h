@@ -408,7 +408,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // 0, which walk_generic looks for, needs a zero direction component.)  Every
 // load is waited for in the block; a mask that a comparison writes goes through
 // a scalar instruction, or two others, before a select reads it.
-#define VRT_WALK(LOAD)                                                                                  \
+#define VRT_WALK(LOAD, COUNT, COUNTED)                                                                  \
     "s_mov_b64 %[ex], exec\n\t"                                                                         \
     "s_and_b64 exec, exec, %[alive]\n\t"                                                                \
     "s_cbranch_execz 9f\n\t"                                                                            \
@@ -424,16 +424,14 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "v_sub_u32_e32 %[idx], %[idx], %[sel]\n\t"                                                          \
     LOAD                                                                                                \
     "v_add_f32_e32 %[trav], 1.0, %[trav]\n\t"                                                           \
-    "v_add_u32_e32 %[iters], 1, %[iters]\n\t"                                                           \
+    COUNT                                                                                               \
     "s_waitcnt vmcnt(0)\n\t"                                                                            \
-    "v_cmp_gt_i32_e32 vcc, 0, %[word]\n\t"                                                              \
-    "s_and_b64 exec, exec, vcc\n\t" /* solid: done */                                                   \
-    "s_cbranch_execz 9f\n\t"                                                                            \
-    "v_cmp_ne_u32_e32 vcc, -1, %[word]\n\t"                                                             \
+    "v_cmp_gt_i32_e32 vcc, -1, %[word]\n\t" /* below -1: jumps */                                       \
     "s_andn2_b64 %[stp], exec, vcc\n\t"                                                                 \
     "s_cbranch_scc0 3f\n\t" /* every lane jumps */                                                      \
-    "s_mov_b64 %[jmp], vcc\n\t" /* a step through a -1 cell: its axis's intersect moves on */           \
-    "s_andn2_b64 exec, %[stp], %[nbx]\n\t"                                                              \
+    "s_mov_b64 %[jmp], vcc\n\t"                                                                         \
+    "v_cmp_eq_u32_e64 %[stp], -1, %[word]\n\t" /* the others are solid: done */                         \
+    "s_andn2_b64 exec, %[stp], %[nbx]\n\t" /* a step through a -1 cell: its axis's intersect moves on */\
     "v_add_f32_e32 %[ix], %[ix], %[ddx]\n\t"                                                            \
     "s_and_b64 %[ta], %[stp], %[nbx]\n\t"                                                               \
     "s_andn2_b64 exec, %[ta], %[nby]\n\t"                                                               \
@@ -543,7 +541,8 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "s_mov_b64 exec, %[jmp]\n\t"                                                                        \
     "s_branch 5b\n\t"                                                                                   \
     "9:\n\t"                                                                                            \
-    "s_mov_b64 exec, %[ex]\n\t"
+    "s_mov_b64 exec, %[ex]\n\t"                                                                         \
+    COUNTED
 
 static_assert((uint32_t)kGuardCorner == 0xffc00001u, "as written in the loop");
 
@@ -558,39 +557,69 @@ struct Walk {
     [sx] "+&v"(w.sx), [sy] "+&v"(w.sy), [sz] "+&v"(w.sz), [ix] "+&v"(w.ix), [iy] "+&v"(w.iy),                   \
         [iz] "+&v"(w.iz), [trav] "+&v"(w.trav), [iters] "+&v"(w.iters), [word] "+&v"(w.word), [ex] "=&s"(ex),   \
         [nbx] "=&s"(nbx), [nby] "=&s"(nby), [stp] "=&s"(stp), [jmp] "=&s"(jmp), [ta] "=&s"(ta),                 \
-        [cur] "=&v"(cur), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [sel] "=&v"(sel)
+        [cur] "=&v"(cur), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [sel] "=&v"(sel), [n] "+&s"(n),       \
+        [k] "=&s"(k)
 #define VRT_WALK_IN                                                                                             \
     [dx] "v"(w.dx), [dy] "v"(w.dy), [dz] "v"(w.dz), [rx] "v"(w.rx), [ry] "v"(w.ry), [rz] "v"(w.rz),             \
         [ddx] "v"(w.ddx), [ddy] "v"(w.ddy), [ddz] "v"(w.ddz), [nstx] "v"(w.nstx), [nsty] "v"(w.nsty),           \
         [nstz] "v"(w.nstz), [lox] "v"(w.lox), [loy] "v"(w.loy), [loz] "v"(w.loz), [base] "v"(w.base),           \
-        [tb] "v"(w.tb), [vox] "s"(vox), [alive] "s"(alive)
+        [tb] "v"(w.tb), [vox] "s"(vox), [alive] "s"(alive), [lim] "v"(lim)
+#define VRT_LOAD_B "global_load_dword %[word], %[idx], %[vox]\n\t"
+// Word indices reach past 4 GiB: the address is 64 bits, from the index in the
+// low half of a register pair whose high half is 0.
+#define VRT_LOAD_32 "v_lshl_add_u64 %[addr], v[4:5], 2, %[vox]\n\tglobal_load_dword %[word], %[addr], off\n\t"
+// Iterations per lane; or their sum over the wave, kept on the scalar unit and
+// left in the first active lane (the others hold 0).
+#define VRT_COUNT_LANES "v_add_u32_e32 %[iters], 1, %[iters]\n\t"
+#define VRT_COUNT_WAVE "s_bcnt1_i32_b64 %[k], exec\n\ts_add_u32 %[n], %[n], %[k]\n\t"
+#define VRT_COUNTED_WAVE \
+    "s_ff1_i32_b64 %[k], exec\n\ts_mov_b32 m0, %[k]\n\ts_nop 0\n\tv_writelane_b32 %[iters], %[n], m0\n\t"
 
-// Runs the loop for the lanes of `alive` until none is left.
+// Runs the loop for the lanes of `alive` until none is left.  kLanes: w.iters
+// counts each lane's iterations; else the wave's sum ends in one lane.
+template <bool kLanes>
 __device__ __forceinline__ void run_walk(IdxB, const int32_t* vox, float lim, uint64_t alive, Walk& w) {
     uint64_t ex, nbx, nby, stp, jmp, ta;
     float cur, t0, t1, t2;
     int32_t sel;
-    asm volatile(VRT_WALK("global_load_dword %[word], %[idx], %[vox]\n\t")
-                 : VRT_WALK_OUT, [idx] "+&v"(w.idx)
-                 : VRT_WALK_IN, [lim] "v"(lim)
-                 : "vcc", "scc", "memory");
+    uint32_t n = 0, k;
+    if constexpr (kLanes)
+        asm volatile(VRT_WALK(VRT_LOAD_B, VRT_COUNT_LANES, "")
+                     : VRT_WALK_OUT, [idx] "+&v"(w.idx)
+                     : VRT_WALK_IN
+                     : "vcc", "scc", "memory");
+    else
+        asm volatile(VRT_WALK(VRT_LOAD_B, VRT_COUNT_WAVE, VRT_COUNTED_WAVE)
+                     : VRT_WALK_OUT, [idx] "+&v"(w.idx)
+                     : VRT_WALK_IN
+                     : "vcc", "scc", "m0", "memory");
 }
-// Word indices reach past 4 GiB: the address is 64 bits, from the index in the
-// low half of a register pair whose high half is 0.
+template <bool kLanes>
 __device__ __forceinline__ void run_walk(Idx32, const int32_t* vox, float lim, uint64_t alive, Walk& w) {
     uint64_t ex, nbx, nby, stp, jmp, ta;
     float cur, t0, t1, t2;
     int32_t sel;
+    uint32_t n = 0, k;
     uint64_t addr;
-    asm volatile(VRT_WALK("v_lshl_add_u64 %[addr], v[4:5], 2, %[vox]\n\t"
-                          "global_load_dword %[word], %[addr], off\n\t")
-                 : VRT_WALK_OUT, [idx] "+&{v4}"(w.idx), [addr] "=&v"(addr)
-                 : VRT_WALK_IN, [lim] "v"(lim), [zero] "{v5}"(0u)
-                 : "vcc", "scc", "memory");
+    if constexpr (kLanes)
+        asm volatile(VRT_WALK(VRT_LOAD_32, VRT_COUNT_LANES, "")
+                     : VRT_WALK_OUT, [idx] "+&{v4}"(w.idx), [addr] "=&v"(addr)
+                     : VRT_WALK_IN, [zero] "{v5}"(0u)
+                     : "vcc", "scc", "memory");
+    else
+        asm volatile(VRT_WALK(VRT_LOAD_32, VRT_COUNT_WAVE, VRT_COUNTED_WAVE)
+                     : VRT_WALK_OUT, [idx] "+&{v4}"(w.idx), [addr] "=&v"(addr)
+                     : VRT_WALK_IN, [zero] "{v5}"(0u)
+                     : "vcc", "scc", "m0", "memory");
 }
 #undef VRT_WALK
 #undef VRT_WALK_OUT
 #undef VRT_WALK_IN
+#undef VRT_LOAD_B
+#undef VRT_LOAD_32
+#undef VRT_COUNT_LANES
+#undef VRT_COUNT_WAVE
+#undef VRT_COUNTED_WAVE
 
 // castRay, src/fshader.glsl:59-129 (see walk_generic for lim), from p, or with
 // kHit from p + d * 0.001 (the shadow rays' start, :152, :165).  ytop: the cutoff's
@@ -603,10 +632,13 @@ __device__ __forceinline__ void run_walk(Idx32, const int32_t* vox, float lim, u
 // inside the grid (any other takes walk_generic).  Else: the reference's
 // formulas.  (The camera's distances to its cell's boundaries made with the
 // frame instead of by every lane: no gain, small frames 2% slower.)
-template <typename IX, bool kHit>
+// kLanes: h.iters is the ray's own iterations (a step map or the depth view
+// shows them); else the lanes' h.iters only add up to the wave's.
+template <typename IX, bool kHit, bool kLanes>
 __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, float pz, float dx, float dy,
                                          float dz, float lim, Hit& h, int32_t ytop) {
     bool general = true;
+    uint32_t counted = 0;  // of the wave's sum, what this lane holds
     if constexpr (!std::is_same_v<IX, Idx64>) {
         const float sx = kHit ? px + dx * 0.001f : px, sy = kHit ? py + dy * 0.001f : py,
                     sz = kHit ? pz + dz * 0.001f : pz;
@@ -680,7 +712,7 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
             w.trav = 0.0f;
             w.iters = 0;
             w.word = -1;
-            run_walk(IX{}, g.vox, lim, __ballot(0.0f < lim), w);
+            run_walk<kLanes>(IX{}, g.vox, lim, __ballot(0.0f < lim), w);
             auto flip = [](int32_t nst, float v) { return nst < 0 ? -v : v; };
             const bool bx = (w.ix < w.iy) & (w.ix < w.iz), by = (w.iy < w.ix) & (w.iy < w.iz);
             const float cur = bx ? w.ix : (by ? w.iy : w.iz);
@@ -693,15 +725,18 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
             h.index = hit ? IX::word(w.idx) : -1;
             h.word = w.word;
             h.iters = w.iters;
+            if constexpr (!kLanes) counted = w.iters;
             general = w.word == kGuardCorner;
             dx = flip(w.nstx, w.dx);
             dy = flip(w.nsty, w.dy);
             dz = flip(w.nstz, w.dz);
         }
     }
-    if (__builtin_expect(general, 0))
+    if (__builtin_expect(general, 0)) {
         walk_generic<IX>(g, kHit ? px + dx * 0.001f : px, kHit ? py + dy * 0.001f : py, kHit ? pz + dz * 0.001f : pz,
                          dx, dy, dz, lim, h, dy >= 0.0f ? ytop : INT32_MAX);
+        h.iters += counted;
+    }
 }
 
 // main(), src/fshader.glsl:131-190, for the fragment at vPos = (vx, vy), pixel
@@ -709,7 +744,8 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
 // (INT32_MAX: none).  What the primary ray decides is stored before the shadow
 // rays are walked, so it holds no registers meanwhile.  The hit's reference
 // index (two integer divisions) is formed only when the target has a hit map.
-template <typename IX>
+// kLanes: see cast_ray.
+template <typename IX, bool kLanes>
 __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& F, const vrt_target& t, int64_t k,
                                             float vx, float vy, int32_t top, uint32_t& rays, uint32_t& iters) {
     const vrt_frame& f = F.f;
@@ -729,7 +765,7 @@ __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& 
     // output of this draw (no depth view, no step map): a ray that stops
     // there misses, as the reference's walk would.
     Hit h;
-    cast_ray<IX, false>(g, f.cam_pos[0], f.cam_pos[1], f.cam_pos[2], d0, d1, d2, F.render_lim, h,
+    cast_ray<IX, false, kLanes>(g, f.cam_pos[0], f.cam_pos[1], f.cam_pos[2], d0, d1, d2, F.render_lim, h,
                         F.primary_cutoff != 0 ? top : INT32_MAX);
     iters = h.iters;
     uint32_t eval = 0, occ = 0;
@@ -750,9 +786,9 @@ __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& 
     }
     if (t.hit) t.hit[k] = hit ? IX::ref_index(g, h.index) : -1;
     if (t.face) t.face[k] = hit ? (uint8_t)(h.axis * 3 + (h.step + 1)) : (uint8_t)VRT_FACE_MISS;
-    if (t.steps) t.steps[k] = h.iters;
+    if (kLanes && t.steps) t.steps[k] = h.iters;
 
-    if (f.view_depth_field == 1) {
+    if (kLanes && f.view_depth_field == 1) {
         const float s = div_small_int((float)h.iters, 100.0f, 1.0f / 100.0f);
         col0 = s;
         col1 = s;
@@ -768,7 +804,7 @@ __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& 
         // sun shadow (:152-156)
         {
             Hit s;
-            cast_ray<IX, true>(g, hx, hy, hz, tlx, tly, tlz, F.render_lim, s, top);
+            cast_ray<IX, true, kLanes>(g, hx, hy, hz, tlx, tly, tlz, F.render_lim, s, top);
             iters += s.iters;
             eval |= 1u;
             if (s.index == -1) {
@@ -820,7 +856,7 @@ __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& 
             float lim = (float)f2i(dist + 1.0f);
             lim = lim < F.render_lim ? lim : F.render_lim;
             Hit s;
-            cast_ray<IX, true>(g, hx, hy, hz, ux1, uy1, uz1, lim, s, top);
+            cast_ray<IX, true, kLanes>(g, hx, hy, hz, ux1, uy1, uz1, lim, s, top);
             iters += s.iters;
             eval |= 2u << i;
             if (s.index == -1) {

@@ -155,10 +155,16 @@ int launch_cast_rays(const GridDesc& g, int64_t n, const float* start, const flo
                      uint8_t* face, uint32_t* steps, hipStream_t s);
 // parts (chunk_tiles 0 only; nullptr: atomics): one entry per 64-pixel pass
 // (batch_items), added into the counters by launch_fold_parts afterwards.
+bool lane_counts(const GridDesc& g, const FrameDesc& f);  // for `lanes`: true if it is for any view
 int launch_render_batch(const GridDesc& g, const ViewDesc* views_dev, int32_t n_views,
-                        int64_t total_tiles, const vrt_batch_config& cfg, int32_t n_workgroups,
+                        int64_t total_tiles, const vrt_batch_config& cfg, bool lanes, int32_t n_workgroups,
                         unsigned int* queue, unsigned long long* counters, unsigned long long* parts,
                         hipStream_t s);
+inline bool lane_counts(const GridDesc& g, const std::vector<ViewDesc>& views) {
+    bool any = false;
+    for (const ViewDesc& v : views) any |= lane_counts(g, v.frame);
+    return any;
+}
 // Entries a hardware-scheduled multi-view launch writes into `parts`, or -1
 // when its counts must go by atomics (a view's render_lim too large for the
 // 32-bit pass sums, or a persistent configuration).

@@ -1,19 +1,8 @@
 // vrt_render.hip — render kernels for gfx950 (wave64).
 //
 //   k_render_plain : one frame; a wave shades one 8x8 screen tile (one ray per
-//                    lane), a 256-thread workgroup four horizontally adjacent
-//                    tiles, in row-major order.  The four share one CU and its
-//                    L1: on an 8 GiB grid, one-wave workgroups (tiles spread
-//                    over CUs) made 4K frames 38% slower, 2x2, 4x2 or 8x1 tile
-//                    groups 3-4% slower (on the 256 MiB grid one-wave groups
-//                    were 2% faster, 2x2 even).  The hardware deals
-//                    workgroups to the 8 XCDs round-robin, so every XCD gets
-//                    an even share of sky, horizon and terrain tiles; giving
-//                    each XCD a contiguous band of rows instead (for L2
-//                    locality) made the XCDs' loads unequal and the frame 29%
-//                    slower.
-//   k_render_views : many views in one launch, four consecutive (view, tile)
-//                    items per workgroup, scheduled by the hardware.
+//                    lane), tiles in row-major order (wave_item).
+//   k_render_views : many views in one launch, scheduled by the hardware.
 //   k_render_batch : many views in one persistent launch; every wave pops
 //                    chunks of (view, tile) work from a device atomic queue
 //                    until the queue is empty (the exit every wave reaches).
@@ -32,9 +21,36 @@ namespace vrt {
 namespace {
 
 constexpr int kWave = 64;
-constexpr int kPlainWaves = 4;                 // waves per workgroup
-constexpr int kPlainThreads = kWave * kPlainWaves;
 constexpr int kXcds = 8;
+
+// Waves per workgroup of the hardware-scheduled kernels.  A 4-wave workgroup
+// starts only when one CU has a slot free on each of its SIMDs, so slots stand
+// empty meanwhile; one-wave workgroups fill them at once.  But the four
+// adjacent tiles of a 4-wave workgroup share a CU's L1, which is worth more
+// where walks spread over a render copy beyond 4 GiB (Idx32, Idx64).  Four waves
+// against one: 1080p in a 256 MiB grid 107.8 and 102.3 us, 1366x768 with all
+// maps 74.3 and 67.9, 3840x2160 in a 1 GiB grid 326 and 319, 320x180 30.0 and
+// 28.8; 3840x2160 in the 8 GiB grid 340 and 358, its depth view 1.39 and 1.95 ms.
+// (Two waves lie between; eight are 18% slower at 1080p.)
+template <typename IX>
+constexpr int kWavesPerGroup = std::is_same_v<IX, dev::IdxB> ? 1 : 4;
+
+// The tile or pass that a wave takes.  Workgroups go to the XCDs round-robin;
+// runs of four items stay on one XCD and its L2 (one-wave workgroups b, b + 8,
+// b + 16, b + 24 of each 32; without that 1366x768 took 72.2 us), so every XCD still gets an even share of sky,
+// horizon and terrain tiles.  (A contiguous band of rows per XCD had the better
+// hit rate but unequal loads, 29% slower.)
+template <typename IX>
+__device__ __forceinline__ uint32_t wave_item() {
+    const uint32_t b = blockIdx.x;
+    if constexpr (kWavesPerGroup<IX> == 1) return ((b / 32) * kXcds + b % kXcds) * 4 + (b / kXcds) % 4;
+    return b * kWavesPerGroup<IX> + (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)(threadIdx.x >> 6));
+}
+// Workgroups for n items.
+template <typename IX>
+int64_t groups_for(int64_t n) {
+    return kWavesPerGroup<IX> == 1 ? (n + 31) / 32 * 32 : (n + kWavesPerGroup<IX> - 1) / kWavesPerGroup<IX>;
+}
 constexpr int kQueueStride = 32;  // queue counters 128 bytes apart
 
 // n / d and n % d for a wave-uniform n, on the scalar unit, from rcp =
@@ -91,15 +107,14 @@ __device__ __forceinline__ void flush_counters_tile(unsigned long long* counters
 // waves_per_eu(8, 8): without it the build ran at 7 resident waves per SIMD
 // (peak measured with per-wave timestamps: 7168 waves on 1024 SIMDs); with it,
 // 8 (a few registers of the rare IEEE-division path spill), 4% faster.
-template <typename IX>
-__global__ void __launch_bounds__(kPlainThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
+template <typename IX, bool kLanes>
+__global__ void __launch_bounds__(kWave * kWavesPerGroup<IX>) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_render_plain(GridDesc g, FrameDesc F, vrt_target t, unsigned long long* counters, unsigned long long* parts) {
     const int32_t top = g.top ? *g.top : INT32_MAX;
-    const uint32_t lb = blockIdx.x;
     const int32_t tiles_x = (t.width + 7) >> 3;
     const int32_t tiles_y = (t.height + 7) >> 3;
     // the wave's tile is uniform: the tile arithmetic runs on the scalar unit
-    const int32_t tile = (int32_t)lb * kPlainWaves + __builtin_amdgcn_readfirstlane((int32_t)(threadIdx.x >> 6));
+    const int32_t tile = (int32_t)wave_item<IX>();
     const int32_t lane = threadIdx.x & 63;
     uint32_t rays = 0, iters = 0, pixels = 0;
     if (tile < tiles_x * tiles_y) {
@@ -112,7 +127,7 @@ k_render_plain(GridDesc g, FrameDesc F, vrt_target t, unsigned long long* counte
         if (px < t.width && row < t.height) {
             float vx, vy;
             dev::pixel_vpos(t.width, t.height, F.inv_w, F.inv_h, px, row, vx, vy);
-            dev::shade_pixel<IX>(g, F, t, (int64_t)row * t.width + px, vx, vy, top, rays, iters);
+            dev::shade_pixel<IX, kLanes>(g, F, t, (int64_t)row * t.width + px, vx, vy, top, rays, iters);
             pixels = 1;
         }
     }
@@ -148,7 +163,7 @@ __global__ void __launch_bounds__(256) k_cast_rays(GridDesc g, int64_t n, const 
     lim = lim < render_lim ? lim : render_lim;
     // the cutoff applies when the caller does not ask for the step counts
     dev::Hit h;
-    dev::cast_ray<IX, false>(g, start[3 * i], start[3 * i + 1], start[3 * i + 2], dir[3 * i], dir[3 * i + 1],
+    dev::cast_ray<IX, false, true>(g, start[3 * i], start[3 * i + 1], start[3 * i + 2], dir[3 * i], dir[3 * i + 1],
                              dir[3 * i + 2], lim, h, steps == nullptr ? top : INT32_MAX);
     const bool hitp = h.index != -1;
     if (hit) hit[i] = hitp ? IX::ref_index(g, h.index) : -1;
@@ -171,7 +186,7 @@ __global__ void __launch_bounds__(256) k_cast_rays(GridDesc g, int64_t n, const 
 // accepts (tiles per launch < 2^32; 18 rays and at most 18 * 2^24 steps a
 // pixel would overflow only past ~14 pixels at the step cap); they are widened
 // when the wave flushes.
-template <typename IX, int TW, int TH>
+template <typename IX, int TW, int TH, bool kLanes>
 __device__ __forceinline__ void shade_view_tile(const GridDesc& g, const ViewDesc* __restrict__ views,
                                                 int32_t n_views, int64_t tile, int32_t first_pass,
                                                 int32_t n_passes, int32_t lane, int32_t top, uint32_t& rays,
@@ -197,7 +212,7 @@ __device__ __forceinline__ void shade_view_tile(const GridDesc& g, const ViewDes
             float vx, vy;
             dev::pixel_vpos(V.target.width, V.target.height, V.frame.inv_w, V.frame.inv_h, px, row, vx, vy);
             uint32_t r, n;
-            dev::shade_pixel<IX>(g, V.frame, V.target, (int64_t)row * V.target.width + px, vx, vy, top, r, n);
+            dev::shade_pixel<IX, kLanes>(g, V.frame, V.target, (int64_t)row * V.target.width + px, vx, vy, top, r, n);
             rays += r;
             iters += n;
             pixels += 1;
@@ -206,24 +221,22 @@ __device__ __forceinline__ void shade_view_tile(const GridDesc& g, const ViewDes
 }
 
 // Multi-view launch scheduled by the hardware.  Every wave shades one pass of
-// 64 pixels: work item i is pass i mod P of tile i / P (P = TW*TH/64), and a
-// 256-thread workgroup takes four consecutive items, so its waves share the
-// CU's L1 over one 16x16 tile or four adjacent smaller ones.  With one pass
-// per wave no value lives across a second walk, which keeps every tile shape
-// within 64 VGPRs without spilling.  The dispatcher hands out workgroups in
-// order as slots free up, so the views' tiles are balanced over the device
-// without any queue.
-template <typename IX, int TW, int TH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
+// 64 pixels: work item i is pass i mod P of tile i / P (P = TW*TH/64; wave_item).
+// With one pass per wave no value lives across a second walk, which keeps every
+// tile shape within 64 VGPRs without spilling.  The dispatcher hands out
+// workgroups in order as slots free up, so the views' tiles are balanced over
+// the device without any queue.
+template <typename IX, int TW, int TH, bool kLanes>
+__global__ void __launch_bounds__(kWave * kWavesPerGroup<IX>) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_render_views(GridDesc g, const ViewDesc* __restrict__ views, int32_t n_views, int64_t total_tiles,
                unsigned long long* counters, unsigned long long* parts) {
     constexpr int32_t kPasses = TW * TH / kWave;
     const int32_t top = g.top ? *g.top : INT32_MAX;
     const int32_t lane = threadIdx.x & 63;
-    const int64_t item = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int32_t)(threadIdx.x >> 6));
+    const int64_t item = (int64_t)wave_item<IX>();
     uint32_t rays = 0, iters = 0, pixels = 0;
     if (item < total_tiles * kPasses)
-        shade_view_tile<IX, TW, TH>(g, views, n_views, item / kPasses, (int32_t)(item % kPasses), 1, lane, top, rays,
+        shade_view_tile<IX, TW, TH, kLanes>(g, views, n_views, item / kPasses, (int32_t)(item % kPasses), 1, lane, top, rays,
                                     iters, pixels);
     if (parts) {
         // one pass of 64 pixels has a tile's bounds; the host passes parts
@@ -245,6 +258,8 @@ k_render_views(GridDesc g, const ViewDesc* __restrict__ views, int32_t n_views, 
 // device-scope atomics on one word per XCD, so they pay off only when tiles
 // are large: on one 1080p frame of 8x8 tiles this kernel ran 50% slower than
 // k_render_views (2.8x slower with a single counter for all XCDs).
+// Iterations are counted lane by lane: a lane's 32-bit count runs over many
+// tiles here, a wave's sum in one lane could overflow it.
 // Held to 8 waves per SIMD, the queue loop's state spills about 28 SGPRs
 // into VGPR lanes and one VGPR to scratch; at the compiler's own budget (67
 // VGPRs, 7 waves, no spill) the 64-view set took 11.7 ms instead of 10.4.
@@ -268,7 +283,7 @@ k_render_batch(GridDesc g, const ViewDesc* __restrict__ views, int32_t n_views, 
             if (base >= r1 - r0) break;
             const uint32_t end = r1 - r0 - base > (uint32_t)chunk ? r0 + base + (uint32_t)chunk : r1;
             for (uint64_t item = (uint64_t)(r0 + base) * kPasses; item < (uint64_t)end * kPasses; item++)
-                shade_view_tile<IX, TW, TH>(g, views, n_views, (int64_t)(item / kPasses), (int32_t)(item % kPasses), 1,
+                shade_view_tile<IX, TW, TH, true>(g, views, n_views, (int64_t)(item / kPasses), (int32_t)(item % kPasses), 1,
                                             lane, top, rays, iters, pixels);
         }
     }
@@ -323,15 +338,29 @@ void with_index(const GridDesc& g, F&& f) {
 
 }  // namespace
 
+// Whether a frame's iterations have to be counted lane by lane (one VALU
+// instruction an iteration more than the wave's sum, which takes two scalar
+// ones): a step map or the depth view shows them, with the cutoff off the total
+// is the reference's to the last one, also where a walk is begun again, and the
+// wave's sum has to fit 32 bits.
+bool lane_counts(const GridDesc& g, const FrameDesc& f) {
+    return f.primary_cutoff == 0 || g.top == nullptr || !(f.render_lim < kTileSum32Lim);
+}
+
 int launch_render_plain(const GridDesc& g, const FrameDesc& f, const vrt_target& t, unsigned long long* counters,
                         unsigned long long* parts, hipStream_t s) {
     const int64_t tiles = (int64_t)((t.width + 7) / 8) * ((t.height + 7) / 8);
-    const int64_t blocks = (tiles + kPlainWaves - 1) / kPlainWaves;
-    if (blocks <= 0) return VRT_OK;
-    if (blocks > 0x7fffffff) return fail(VRT_ERR_INVALID, "frame too large");
+    if (tiles <= 0) return VRT_OK;
+    if (tiles > 0x7fffffe0) return fail(VRT_ERR_INVALID, "frame too large");
     with_index(g, [&](auto ix) {
-        hipLaunchKernelGGL(k_render_plain<decltype(ix)>, dim3((uint32_t)blocks), dim3(kPlainThreads), 0, s, g, f, t,
-                           counters, parts);
+        // The wave's sum is the faster count where VALU issue is the bound (64
+        // views in one launch 5.76 -> 5.68 ms, 3840x2160 346 -> 341 us), not
+        // where a frame has less than about two tiles for each of the 8,192
+        // wave slots and waits for its longest walk (320x180: 30.0 -> 30.3 us).
+        const bool lanes = lane_counts(g, f) || tiles <= 16384;
+        auto* kernel = lanes ? k_render_plain<decltype(ix), true> : k_render_plain<decltype(ix), false>;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)groups_for<decltype(ix)>(tiles)),
+                           dim3(kWave * kWavesPerGroup<decltype(ix)>), 0, s, g, f, t, counters, parts);
     });
     VRT_HIP(hipGetLastError());
     return VRT_OK;
@@ -381,18 +410,21 @@ int batch_occupancy(const vrt_batch_config& cfg, int32_t* waves_per_cu) {
 }
 
 int launch_render_batch(const GridDesc& g, const ViewDesc* views_dev, int32_t n_views, int64_t total_tiles,
-                        const vrt_batch_config& cfg, int32_t n_workgroups, unsigned int* queue,
+                        const vrt_batch_config& cfg, bool lanes, int32_t n_workgroups, unsigned int* queue,
                         unsigned long long* counters, unsigned long long* parts, hipStream_t s) {
     if (parts && cfg.chunk_tiles != 0) return fail(VRT_ERR_INVALID, "partial counts need the hardware-scheduled kernel");
     if (cfg.chunk_tiles == 0) {
-        const int64_t wgs = (total_tiles * (cfg.tile_w * cfg.tile_h / 64) + 3) / 4;  // one wave per 64 pixels
-        if (wgs <= 0) return VRT_OK;
-        if (wgs > 0x7fffffff) return fail(VRT_ERR_INVALID, "too many tiles in one batch");
+        const int64_t items = total_tiles * (cfg.tile_w * cfg.tile_h / 64);  // one wave per 64 pixels
+        if (items <= 0) return VRT_OK;
+        if (items > 0x7fffffe0) return fail(VRT_ERR_INVALID, "too many tiles in one batch");
         if (int rc = with_shape(cfg.tile_w, cfg.tile_h, [&](auto tw, auto th) {
                 with_index(g, [&](auto ix) {
-                    hipLaunchKernelGGL((k_render_views<decltype(ix), decltype(tw)::value, decltype(th)::value>),
-                                       dim3((uint32_t)wgs), dim3(256), 0, s, g, views_dev, n_views, total_tiles,
-                                       counters, parts);
+                    constexpr int TW = decltype(tw)::value, TH = decltype(th)::value;
+                    auto* kernel =
+                        lanes ? k_render_views<decltype(ix), TW, TH, true> : k_render_views<decltype(ix), TW, TH, false>;
+                    const int64_t wgs = groups_for<decltype(ix)>(items);
+                    hipLaunchKernelGGL(kernel, dim3((uint32_t)wgs), dim3(kWave * kWavesPerGroup<decltype(ix)>), 0, s,
+                                       g, views_dev, n_views, total_tiles, counters, parts);
                 });
             }))
             return rc;
