@@ -236,9 +236,9 @@ struct Idx64 {
 // computed with selects so the wave does not branch.
 //
 // ytop (shadow rays, and primary rays whose step count nothing shows): an
-// upper bound on the y of every solid voxel, or INT32_MAX.  Let dy >= 0.  Every cell of a segment has y >= int(start.y),
-// and a jump sets start.y += RN(dy * c) with c = the entry intersect plus the
-// jump.  A negative entry intersect either belongs to an axis whose step
+// upper bound on the y of every solid voxel, or INT32_MAX.  Let dy >= 0.  Every
+// cell of a segment has y >= int(start.y), and a jump sets start.y += RN(dy * c)
+// with c = the entry intersect plus the jump.  A negative entry intersect either belongs to an axis whose step
 // leaves the grid (the walk ends before any jump), or comes from a zero
 // direction component, which then makes c infinite or NaN at every jump from
 // the first one on.  So after a jump that leaves int(start.y) > ytop with c
@@ -249,9 +249,11 @@ struct Idx64 {
 // with c = -inf or NaN leaves int(start.y) at INT32_MIN or 0, where the test
 // fires only if the grid has no solid voxel; c = +inf makes `travelled`
 // infinite, which ends the walk at the next loop test anyway.)
-template <typename IX>
+// kAgain: where `again`, the walk is one that run_walk gave up, whose iterations
+// are counted already up to there; h.iters leaves these out.
+template <typename IX, bool kAgain>
 __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float sy, float sz, float dx, float dy,
-                                         float dz, float lim, Hit& h, int32_t ytop) {
+                                             float dz, float lim, Hit& h, int32_t ytop, bool again) {
     using T = typename IX::T;
     const int32_t cx = f2i(sx), cy = f2i(sy), cz = f2i(sz);
     const int32_t stx = isign(dx), sty = isign(dy), stz = isign(dz);
@@ -289,7 +291,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     const int32_t* __restrict__ vox = g.vox;
 
     float trav = 0.0f;
-    uint32_t iters = 0;
+    uint32_t iters = 0, counted = 0;
     int32_t axis = -1;
     int64_t result = -1;
     while (trav < lim) {
@@ -326,6 +328,17 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
             // jump recomputes is read after that.  One branch for that and
             // the cutoff.
             if (!(trav < lim) | (cy > ytop)) break;
+            if constexpr (kAgain) {
+                // run_walk's two ends: a tiny fraction at a jump, or the step
+                // after a jump to below both x = 0 and y = 0
+                const bool tiny = ((sx > 0.0f) & (sx < 0x1p-60f)) | ((sy > 0.0f) & (sy < 0x1p-60f)) |
+                                  ((sz > 0.0f) & (sz < 0x1p-60f));
+                const bool edge = (sx < 0.0f) & (sy < 0.0f);
+                if (again & (tiny | edge)) {
+                    counted = iters + (tiny ? 0 : 1);
+                    again = false;
+                }
+            }
             div3_by((float)(cx + fx) - sx, (float)(cy + fy) - sy, (float)(cz + fz) - sz, dx, dy, dz, rx, ry, rz, dok,
                     ix, iy, iz);
             idx = IX::make(g, clamp_cell(cx, g.X), clamp_cell(cy, g.Y), clamp_cell(cz, g.Z));
@@ -357,15 +370,16 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     h.index = result;
     h.axis = axis;
     h.step = axis == 0 ? stx : (axis == 1 ? sty : stz);
-    h.iters = iters;
+    h.iters = kAgain ? iters - counted : iters;
 }
 
 // The same walk for 32-bit indices (IdxB, Idx32), where it is bound by VALU
 // issue: its loop is written out, with the arithmetic arranged so that a jump
-// takes 34 VALU instructions instead of 41, a step 4 instead of 7, and an
-// iteration 8 scalar ones where the compiler's loop has 24.  1920x1080, sun and
-// 16 lights: 152 -> 121 us; 3840x2160 in the 8 GiB grid: 491 -> 407 us; 64 views
-// in one launch: 7.64 -> 6.25 ms; 320x180 (one walk's latency): 30.6 -> 26.3 us.
+// takes 35 VALU instructions instead of 41, a step 5 instead of 7, and an
+// iteration 8 scalar ones where the compiler's loop has 24.  Against the
+// compiler's loop, all else alike, 1920x1080 with sun and 16 lights: 152 -> 121
+// us; 3840x2160 in the 8 GiB grid: 491 -> 407 us; 64 views in one launch: 7.64
+// -> 6.25 ms; 320x180 (one walk's latency): 30.6 -> 26.3 us.
 //
 // Mirrored axes.  Negating a position and a direction component together
 // negates every product and sum of the walk exactly (rounding to nearest is
@@ -378,11 +392,12 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // takes up the 1.
 //
 // Which rays: those whose direction components lie in [2^-19, 2^60] in
-// magnitude and whose start coordinates lie in [2^-20, 2^22] (cast_ray).  On an ascending axis s then stays at least 2^-20, where the
-// hardware's fraction is the rounded difference; on a descending one s may
-// fall below 0 only on its way out of the grid (below).  Only the low end of a
-// cell is clamped (lo: clamp_cell's -2 or n + 1, mirrored): a ray jumps from
-// inside the grid, downward on every axis.
+// magnitude and whose start coordinates lie in [2^-20, 2^22] (cast_ray).  On an
+// ascending axis s then stays at least 2^-20, where the hardware's fraction is
+// the rounded difference; on a descending one s may fall below 0 only on its
+// way out of the grid (below).  Only the low end of a cell is clamped (lo:
+// clamp_cell's -2 or n + 1, mirrored): a ray jumps from inside the grid,
+// downward on every axis.
 //
 // After a jump a fraction may be below 2^-60, where the quotient's three
 // instructions are not exact (label 6).  Where s is whole it is 0, and the
@@ -455,7 +470,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "v_add_f32_e32 %[sz], %[t2], %[sz]\n\t"                                                             \
     "v_cvt_flr_i32_f32_e32 %[t1], %[sy]\n\t"                                                            \
     "v_cmp_gt_f32_e32 vcc, %[lim], %[trav]\n\t"                                                         \
-    "v_cmp_ge_i32_e64 %[ta], %[t1], %[tb]\n\t"                                                          \
+    "v_cmp_gt_f32_e64 %[ta], %[sy], %[tb]\n\t"                                                          \
     "s_and_b64 exec, vcc, %[ta]\n\t" /* out of budget or grid, or above the solid top: a miss */        \
     "s_cbranch_execz 5f\n\t"                                                                            \
     "v_fract_f32_e32 %[ix], %[sx]\n\t"                                                                  \
@@ -550,7 +565,8 @@ static_assert((uint32_t)kGuardCorner == 0xffc00001u, "as written in the loop");
 struct Walk {
     float sx, sy, sz, dx, dy, dz, rx, ry, rz, ddx, ddy, ddz, ix, iy, iz, trav;
     uint32_t idx, base, iters;
-    int32_t nstx, nsty, nstz, lox, loy, loz, tb, word;
+    int32_t nstx, nsty, nstz, lox, loy, loz, word;
+    float tb;
 };
 
 #define VRT_WALK_OUT                                                                                            \
@@ -621,6 +637,89 @@ __device__ __forceinline__ void run_walk(Idx32, const int32_t* vox, float lim, u
 #undef VRT_COUNT_WAVE
 #undef VRT_COUNTED_WAVE
 
+// The walk's state at a ray's start (arguments as cast_ray's), for rays that
+// run_walk takes; false for any other.
+//
+// The first cell and intersects.  From a hit: as after a jump, for a start
+// inside the grid (any other takes walk_generic).  Else: the reference's
+// formulas.  (The camera's distances to its cell's boundaries made with the
+// frame instead of by every lane: no gain, small frames 2% slower.)
+template <typename IX, bool kHit>
+__device__ __forceinline__ bool start_walk(const GridDesc& g, float px, float py, float pz, float dx, float dy,
+                                           float dz, Walk& w) {
+    const float sx = kHit ? px + dx * 0.001f : px, sy = kHit ? py + dy * 0.001f : py,
+                sz = kHit ? pz + dz * 0.001f : pz;
+    const bool mx = dx > 0.0f, my = dy > 0.0f, mz = dz > 0.0f;
+    w.sx = mx ? -sx : sx;
+    w.sy = my ? -sy : sy;
+    w.sz = mz ? -sz : sz;
+    // |d| >= 2^-19 keeps |d + 1e-6| in range too.  min and max pass over a
+    // NaN; the comparisons of s (NaN where d is) or the sum do not.
+    const float lo = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
+    const float hi = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz));
+    bool fast = (lo >= 0x1p-19f) & (hi <= 0x1p60f);
+    if constexpr (kHit) {
+        w.ix = __builtin_amdgcn_fractf(w.sx);
+        w.iy = __builtin_amdgcn_fractf(w.sy);
+        w.iz = __builtin_amdgcn_fractf(w.sz);
+        fast &= (fminf(fminf(sx, sy), sz) >= 0x1p-20f) & (sx < g.FX) & (sy < g.FY) & (sz < g.FZ);
+    } else {
+        const float sum = ((dx + dy) + dz) + ((sx + sy) + sz);
+        fast &= (fminf(fminf(sx, sy), sz) >= 0x1p-20f) & (fmaxf(fmaxf(sx, sy), sz) <= 0x1p22f) & (sum == sum);
+    }
+    if (!fast) return false;
+    w.ddx = rcp_fast(fabsf(dx + 0.000001f));
+    w.ddy = rcp_fast(fabsf(dy + 0.000001f));
+    w.ddz = rcp_fast(fabsf(dz + 0.000001f));
+    w.rx = rcp_fast(fabsf(dx));
+    w.ry = rcp_fast(fabsf(dy));
+    w.rz = rcp_fast(fabsf(dz));
+    w.dx = -fabsf(dx);
+    w.dy = -fabsf(dy);
+    w.dz = -fabsf(dz);
+    w.nstx = (int32_t)IX::stride(g, mx ? -1 : 1, 0);
+    w.nsty = (int32_t)IX::stride(g, my ? -1 : 1, 1);
+    w.nstz = (int32_t)IX::stride(g, mz ? -1 : 1, 2);
+    w.lox = mx ? -(int32_t)g.X - 2 : -2;
+    w.loy = my ? -(int32_t)g.Y - 2 : -2;
+    w.loz = mz ? -(int32_t)g.Z - 2 : -2;
+    w.base = IX::make(g, 0, 0, 0) + (uint32_t)((mx ? w.nstx : 0) + (my ? w.nsty : 0) + (mz ? w.nstz : 0));
+    if constexpr (kHit) {
+        // u / |d| as after a jump: exact for u = 0 and u >= 2^-60
+        auto quotient = [](float u, float d, float r) {
+            const float q0 = u * r;
+            return __builtin_fmaf(__builtin_fmaf(q0, d, u), r, q0);
+        };
+        w.idx = IX::add(w.base, floor_i(w.sx), w.nstx);
+        w.idx = IX::add(w.idx, floor_i(w.sy), w.nsty);
+        w.idx = IX::add(w.idx, floor_i(w.sz), w.nstz);
+        // s >= 2^-20, so a fraction is 0 or at least 2^-43.  A whole s
+        // on an ascending axis: the boundary ahead is 1 away, the
+        // cell one lower than floor(s') says.  (Common: a face's
+        // coordinate stays whole where d * 0.001 rounds away.)
+        if (fminf(fminf(w.ix, w.iy), w.iz) == 0.0f) {
+            const bool ax = mx & (w.ix == 0.0f), ay = my & (w.iy == 0.0f), az = mz & (w.iz == 0.0f);
+            w.idx -= (uint32_t)((ax ? w.nstx : 0) + (ay ? w.nsty : 0) + (az ? w.nstz : 0));
+            w.ix = ax ? 1.0f : w.ix;
+            w.iy = ay ? 1.0f : w.iy;
+            w.iz = az ? 1.0f : w.iz;
+        }
+        w.ix = quotient(w.ix, w.dx, w.rx);
+        w.iy = quotient(w.iy, w.dy, w.ry);
+        w.iz = quotient(w.iz, w.dz, w.rz);
+    } else {
+        const int32_t cx = f2i(sx), cy = f2i(sy), cz = f2i(sz);
+        w.idx = IX::make(g, clamp_cell(cx, g.X), clamp_cell(cy, g.Y), clamp_cell(cz, g.Z));
+        div3_by((float)(mx ? -cx - 1 : cx) - w.sx, (float)(my ? -cy - 1 : cy) - w.sy,
+                (float)(mz ? -cz - 1 : cz) - w.sz, w.dx, w.dy, w.dz, -w.rx, -w.ry, -w.rz, true, w.ix, w.iy,
+                w.iz);
+    }
+    w.trav = 0.0f;
+    w.iters = 0;
+    w.word = -1;
+    return true;
+}
+
 // castRay, src/fshader.glsl:59-129 (see walk_generic for lim), from p, or with
 // kHit from p + d * 0.001 (the shadow rays' start, :152, :165).  ytop: the cutoff's
 // bound for a ray that does not head down (INT32_MAX: none).  What the
@@ -628,90 +727,17 @@ __device__ __forceinline__ void run_walk(Idx32, const int32_t* vox, float lim, u
 // steps from d' and the strides, the start from p) rather than held in
 // registers meanwhile.
 //
-// The first cell and intersects.  From a hit: as after a jump, for a start
-// inside the grid (any other takes walk_generic).  Else: the reference's
-// formulas.  (The camera's distances to its cell's boundaries made with the
-// frame instead of by every lane: no gain, small frames 2% slower.)
 // kLanes: h.iters is the ray's own iterations (a step map or the depth view
 // shows them); else the lanes' h.iters only add up to the wave's.
 template <typename IX, bool kHit, bool kLanes>
 __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, float pz, float dx, float dy,
                                          float dz, float lim, Hit& h, int32_t ytop) {
-    bool general = true;
-    uint32_t counted = 0;  // of the wave's sum, what this lane holds
+    bool general = true, again = false;
+    h.iters = 0;
     if constexpr (!std::is_same_v<IX, Idx64>) {
-        const float sx = kHit ? px + dx * 0.001f : px, sy = kHit ? py + dy * 0.001f : py,
-                    sz = kHit ? pz + dz * 0.001f : pz;
         Walk w;
-        const bool mx = dx > 0.0f, my = dy > 0.0f, mz = dz > 0.0f;
-        w.sx = mx ? -sx : sx;
-        w.sy = my ? -sy : sy;
-        w.sz = mz ? -sz : sz;
-        // |d| >= 2^-19 keeps |d + 1e-6| in range too.  min and max pass over a
-        // NaN; the comparisons of s (NaN where d is) or the sum do not.
-        const float lo = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
-        const float hi = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz));
-        bool fast = (lo >= 0x1p-19f) & (hi <= 0x1p60f);
-        if constexpr (kHit) {
-            w.ix = __builtin_amdgcn_fractf(w.sx);
-            w.iy = __builtin_amdgcn_fractf(w.sy);
-            w.iz = __builtin_amdgcn_fractf(w.sz);
-            fast &= (fminf(fminf(sx, sy), sz) >= 0x1p-20f) & (sx < g.FX) & (sy < g.FY) & (sz < g.FZ);
-        } else {
-            const float sum = ((dx + dy) + dz) + ((sx + sy) + sz);
-            fast &= (fminf(fminf(sx, sy), sz) >= 0x1p-20f) & (fmaxf(fmaxf(sx, sy), sz) <= 0x1p22f) & (sum == sum);
-        }
-        if (fast) {
-            w.ddx = rcp_fast(fabsf(dx + 0.000001f));
-            w.ddy = rcp_fast(fabsf(dy + 0.000001f));
-            w.ddz = rcp_fast(fabsf(dz + 0.000001f));
-            w.rx = rcp_fast(fabsf(dx));
-            w.ry = rcp_fast(fabsf(dy));
-            w.rz = rcp_fast(fabsf(dz));
-            w.dx = -fabsf(dx);
-            w.dy = -fabsf(dy);
-            w.dz = -fabsf(dz);
-            w.nstx = (int32_t)IX::stride(g, mx ? -1 : 1, 0);
-            w.nsty = (int32_t)IX::stride(g, my ? -1 : 1, 1);
-            w.nstz = (int32_t)IX::stride(g, mz ? -1 : 1, 2);
-            w.lox = mx ? -(int32_t)g.X - 2 : -2;
-            w.loy = my ? -(int32_t)g.Y - 2 : -2;
-            w.loz = mz ? -(int32_t)g.Z - 2 : -2;
-            w.base = IX::make(g, 0, 0, 0) + (uint32_t)((mx ? w.nstx : 0) + (my ? w.nsty : 0) + (mz ? w.nstz : 0));
-            if constexpr (kHit) {
-                // u / |d| as after a jump: exact for u = 0 and u >= 2^-60
-                auto quotient = [](float u, float d, float r) {
-                    const float q0 = u * r;
-                    return __builtin_fmaf(__builtin_fmaf(q0, d, u), r, q0);
-                };
-                w.idx = IX::add(w.base, floor_i(w.sx), w.nstx);
-                w.idx = IX::add(w.idx, floor_i(w.sy), w.nsty);
-                w.idx = IX::add(w.idx, floor_i(w.sz), w.nstz);
-                // s >= 2^-20, so a fraction is 0 or at least 2^-43.  A whole s
-                // on an ascending axis: the boundary ahead is 1 away, the
-                // cell one lower than floor(s') says.  (Common: a face's
-                // coordinate stays whole where d * 0.001 rounds away.)
-                if (fminf(fminf(w.ix, w.iy), w.iz) == 0.0f) {
-                    const bool ax = mx & (w.ix == 0.0f), ay = my & (w.iy == 0.0f), az = mz & (w.iz == 0.0f);
-                    w.idx -= (uint32_t)((ax ? w.nstx : 0) + (ay ? w.nsty : 0) + (az ? w.nstz : 0));
-                    w.ix = ax ? 1.0f : w.ix;
-                    w.iy = ay ? 1.0f : w.iy;
-                    w.iz = az ? 1.0f : w.iz;
-                }
-                w.ix = quotient(w.ix, w.dx, w.rx);
-                w.iy = quotient(w.iy, w.dy, w.ry);
-                w.iz = quotient(w.iz, w.dz, w.rz);
-            } else {
-                const int32_t cx = f2i(sx), cy = f2i(sy), cz = f2i(sz);
-                w.idx = IX::make(g, clamp_cell(cx, g.X), clamp_cell(cy, g.Y), clamp_cell(cz, g.Z));
-                div3_by((float)(mx ? -cx - 1 : cx) - w.sx, (float)(my ? -cy - 1 : cy) - w.sy,
-                        (float)(mz ? -cz - 1 : cz) - w.sz, w.dx, w.dy, w.dz, -w.rx, -w.ry, -w.rz, true, w.ix, w.iy,
-                        w.iz);
-            }
-            w.tb = my ? -1 - ytop : INT32_MIN;
-            w.trav = 0.0f;
-            w.iters = 0;
-            w.word = -1;
+        if (start_walk<IX, kHit>(g, px, py, pz, dx, dy, dz, w)) {
+            w.tb = dy > 0.0f ? -1.0f - (float)ytop : -__builtin_inff();
             run_walk<kLanes>(IX{}, g.vox, lim, __ballot(0.0f < lim), w);
             auto flip = [](int32_t nst, float v) { return nst < 0 ? -v : v; };
             const bool bx = (w.ix < w.iy) & (w.ix < w.iz), by = (w.iy < w.ix) & (w.iy < w.iz);
@@ -724,18 +750,19 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
             h.step = (bx ? w.nstx : (by ? w.nsty : w.nstz)) < 0 ? 1 : -1;
             h.index = hit ? IX::word(w.idx) : -1;
             h.word = w.word;
-            h.iters = w.iters;
-            if constexpr (!kLanes) counted = w.iters;
-            general = w.word == kGuardCorner;
+            general = again = w.word == kGuardCorner;
             dx = flip(w.nstx, w.dx);
             dy = flip(w.nsty, w.dy);
             dz = flip(w.nstz, w.dz);
+            h.iters = w.iters;
         }
     }
     if (__builtin_expect(general, 0)) {
-        walk_generic<IX>(g, kHit ? px + dx * 0.001f : px, kHit ? py + dy * 0.001f : py, kHit ? pz + dz * 0.001f : pz,
-                         dx, dy, dz, lim, h, dy >= 0.0f ? ytop : INT32_MAX);
-        h.iters += counted;
+        const uint32_t sum = kLanes ? 0 : h.iters;  // of the wave's sum, what this lane holds
+        walk_generic<IX, !kLanes && !std::is_same_v<IX, Idx64>>(
+            g, kHit ? px + dx * 0.001f : px, kHit ? py + dy * 0.001f : py, kHit ? pz + dz * 0.001f : pz, dx, dy, dz, lim, h,
+            dy >= 0.0f ? ytop : INT32_MAX, again);
+        h.iters += sum;
     }
 }
 
@@ -920,7 +947,6 @@ __device__ __forceinline__ unsigned long long wave_sum_u58(unsigned long long v)
     const uint32_t hi = wave_sum_u32((uint32_t)(v >> 26));
     return (unsigned long long)lo + ((unsigned long long)hi << 26);
 }
-
 
 }  // namespace dev
 }  // namespace vrt

@@ -24,7 +24,7 @@ constexpr int32_t kNoAllocMaxViews = 256;
 constexpr size_t kViewBytes = sizeof(ViewDesc) * (size_t)kNoAllocMaxViews;
 constexpr size_t kQueueOffset = (kViewBytes + 255) & ~(size_t)255;
 constexpr size_t kScratchBytes = kQueueOffset + kQueueBytes;
-constexpr int32_t kPutPerLaunch = 4;  // 4 x 912 B of kernel arguments
+constexpr int32_t kPutPerLaunch = 4;  // 4 x 984 B of kernel arguments
 constexpr int32_t kMaxDevices = 64;
 
 // The descriptors and queue counters of vrt_draw_views_noalloc, per GPU.

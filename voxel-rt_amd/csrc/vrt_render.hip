@@ -37,9 +37,9 @@ constexpr int kWavesPerGroup = std::is_same_v<IX, dev::IdxB> ? 1 : 4;
 
 // The tile or pass that a wave takes.  Workgroups go to the XCDs round-robin;
 // runs of four items stay on one XCD and its L2 (one-wave workgroups b, b + 8,
-// b + 16, b + 24 of each 32; without that 1366x768 took 72.2 us), so every XCD still gets an even share of sky,
-// horizon and terrain tiles.  (A contiguous band of rows per XCD had the better
-// hit rate but unequal loads, 29% slower.)
+// b + 16, b + 24 of each 32; without that 1366x768 took 72.2 us), so every XCD
+// still gets an even share of sky, horizon and terrain tiles.  (A contiguous
+// band of rows per XCD had the better hit rate but unequal loads, 29% slower.)
 template <typename IX>
 __device__ __forceinline__ uint32_t wave_item() {
     const uint32_t b = blockIdx.x;
@@ -260,9 +260,9 @@ k_render_views(GridDesc g, const ViewDesc* __restrict__ views, int32_t n_views, 
 // k_render_views (2.8x slower with a single counter for all XCDs).
 // Iterations are counted lane by lane: a lane's 32-bit count runs over many
 // tiles here, a wave's sum in one lane could overflow it.
-// Held to 8 waves per SIMD, the queue loop's state spills about 28 SGPRs
-// into VGPR lanes and one VGPR to scratch; at the compiler's own budget (67
-// VGPRs, 7 waves, no spill) the 64-view set took 11.7 ms instead of 10.4.
+// Held to 8 waves per SIMD, the queue loop's state spills about 40 SGPRs into
+// VGPR lanes and up to five VGPRs to scratch, outside the walk's loop; with 7
+// waves and no spill the 64-view set was 12% slower.
 template <typename IX, int TW, int TH>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_render_batch(GridDesc g, const ViewDesc* __restrict__ views, int32_t n_views, int64_t total_tiles, int32_t chunk,
@@ -340,9 +340,9 @@ void with_index(const GridDesc& g, F&& f) {
 
 // Whether a frame's iterations have to be counted lane by lane (one VALU
 // instruction an iteration more than the wave's sum, which takes two scalar
-// ones): a step map or the depth view shows them, with the cutoff off the total
-// is the reference's to the last one, also where a walk is begun again, and the
-// wave's sum has to fit 32 bits.
+// ones): a step map or the depth view shows them, and the wave's sum has to fit
+// 32 bits.  (primary_cutoff is 0 with a step map, in the depth view, and with the
+// cutoff switched off, where totals are compared with the reference's.)
 bool lane_counts(const GridDesc& g, const FrameDesc& f) {
     return f.primary_cutoff == 0 || g.top == nullptr || !(f.render_lim < kTileSum32Lim);
 }
