@@ -130,6 +130,27 @@ def test_host_matrix_helpers_equal_glm(vrt, probe):
         assert [f32_bits(float(x)) for x in e] == o
 
 
+# ------------------------------------- closed forms that need no GLM sources
+def test_normalize_scales_by_the_reciprocal_length(orc):
+    """normalize(v) is v times the rounded 1 / length(v), as GLM and GLSL state
+    it, not v / length(v): the two differ in the last bit for many v."""
+    rng = np.random.default_rng(4)
+    for v in _rand_vecs(rng, 300):
+        inv = np.float32(1.0) / np.float32(orc.length(v))
+        assert [f32_bits(x) for x in orc.normalize(v)] == [f32_bits(x) for x in v * inv]
+
+
+def test_aspect_ratio_widens_x(orc, vrt):
+    """With the identity for a camera the ray through (x, y) has slopes
+    x * aspect / focal and y / focal, each within a few roundings."""
+    for aspect in (1.0, 16 / 9, 0.5):
+        f = vrt.frame_defaults(512, 1920, 1080)
+        f.aspect_ratio, f.focal = aspect, 1.5
+        f.rotate_matrix[:] = np.eye(4, dtype=np.float32).ravel().tolist()
+        d = orc.primary_dir(f, 0.25, -0.75)
+        assert abs(d[0] / d[2] - 0.25 * aspect / 1.5) < 1e-6 and abs(d[1] / d[2] + 0.75 / 1.5) < 1e-6
+
+
 # -------------------------------------------------------- traversal closed forms
 def empty_grid(dims):
     return np.full(dims[0] * dims[1] * dims[2], -1, np.int32)
