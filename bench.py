@@ -109,9 +109,10 @@ def plain_bench(vrt, steps, warmup, cutoff_off_leg=True):
     ctx.build_depth_field()
     ctx.sync()
     log("1080p world %s, depth field %.3f s" % (sc.dims, time.time() - t0))
-    # One device-to-device copy of the whole grid (256 MiB read + 256 MiB
-    # written by k_copy): a plain copy of known size that calibrates the
-    # profiler's FETCH_SIZE / WRITE_SIZE counters for this run.
+    # One upload of the whole grid from device memory (k_load_grid: 256 MiB
+    # read, 256 MiB of grid and 256 MiB of render copy written): a streaming pass
+    # of known size that calibrates the profiler's FETCH_SIZE / WRITE_SIZE
+    # counters for this run.
     snapshot = vrt.DeviceBuffer(4 * sc.world.size)
     vrt.hip_check(vrt.hip().hipMemcpy(snapshot.ptr, vrt.C.c_void_p(grid_ptr(vrt, ctx)), snapshot.nbytes, vrt.D2D),
                   "hipMemcpy D2D")
