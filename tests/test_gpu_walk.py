@@ -1,6 +1,7 @@
 """The written-out walk (vrt_device.h: cast_ray, run_walk) where its arithmetic
 differs in form from the shader's: whole coordinates after a jump, ties, walks
-that leave the grid by a low face or by the x-y edge, starts outside its range.
+that leave the grid by a low face or by the x-y edge, starts outside its range,
+directions so long that a jump ends beyond 2^31.
 Against the oracle's castRay, bit for bit, for 32-bit byte offsets and 32-bit
 indices."""
 import numpy as np
@@ -84,3 +85,27 @@ def test_leaving_by_the_edge_with_equal_intersects(gpu, orc):
         r = compare(gpu, orc, w, dims, start, np.repeat(np.array([d]), n, 0), np.full(n, 200))
         hits += int((r["hit"][::2] >= 0).sum())
     assert hits == 6 * 35, hits  # every such ray reaches its voxel
+
+
+def jumps_and_solids(rng, dims):
+    cells = dims[0] * dims[1] * dims[2]
+    world = np.full(cells, -1, np.int32)
+    jump = rng.random(cells) < 0.5
+    world[jump] = (-0.5 * rng.integers(1, 17, int(jump.sum())).astype(np.float32)).view(np.int32)
+    solid = rng.random(cells) < 0.04
+    world[solid] = rng.integers(0, 1 << 24, int(solid.sum()))
+    return world
+
+
+@pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
+@pytest.mark.parametrize("axis", [0, 2], ids=["x", "z"])
+def test_long_directions(gpu, orc, dims, axis):
+    """One component of 2^20 to 2^60: most jumps end far outside the grid, many
+    beyond 2^31, where the cell saturates; the walk has to leave the grid there."""
+    rng = np.random.default_rng(40 + axis)
+    world = jumps_and_solids(rng, dims)
+    n = 40000
+    start = np.stack([rng.uniform(0.01, min(s, 48), n) for s in dims], 1)
+    d = rng.choice([-1.0, 1.0], (n, 3)) * 2.0 ** rng.uniform(-8, 2, (n, 3))
+    d[:, axis] = rng.choice([-1.0, 1.0], n) * 2.0 ** rng.uniform(20, 60, n)
+    compare(gpu, orc, world, dims, start, d, rng.integers(1, 200, n))

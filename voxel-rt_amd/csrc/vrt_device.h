@@ -405,7 +405,9 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // ascending one (the quotient RN(1/|d|)), whose cell is then one lower than
 // floor(s') says.  A tiny fraction that is not 0 takes the ray to
 // walk_generic.  (s beyond 2^23 is whole, and outside any grid with 32-bit
-// indices.)
+// indices.  Beyond 2^31, where only directions longer than a unit vector reach,
+// floor(s') is INT32_MIN and the subtraction saturates: wrapped round to
+// INT32_MAX it would pass the clamp, and its low 24 bits are cell 0.)
 //
 // Leaving through a low face.  For -1 < s < 0 the reference's cell is 0, with
 // a negative intersect that its next step takes at once, out of the grid; here
@@ -518,7 +520,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "s_and_b64 %[ta], %[ta], %[nbx]\n\t"                                                                \
     "v_cndmask_b32_e64 %[ix], %[ix], %[rx], %[ta]\n\t"                                                  \
     "v_cndmask_b32_e64 %[t2], 0, 1, %[ta]\n\t"                                                          \
-    "v_sub_u32_e32 %[t1], %[t1], %[t2]\n\t"                                                             \
+    "v_sub_i32 %[t1], %[t1], %[t2] clamp\n\t"                                                           \
     "v_max_i32_e32 %[t1], %[t1], %[lox]\n\t"                                                            \
     "v_mad_i32_i24 %[idx], %[t1], %[nstx], %[idx]\n\t"                                                  \
     "v_fract_f32_e32 %[t0], %[sy]\n\t"                                                                  \
@@ -534,7 +536,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "s_and_b64 %[ta], %[ta], %[nbx]\n\t"                                                                \
     "v_cndmask_b32_e64 %[iy], %[iy], %[ry], %[ta]\n\t"                                                  \
     "v_cndmask_b32_e64 %[t2], 0, 1, %[ta]\n\t"                                                          \
-    "v_sub_u32_e32 %[t1], %[t1], %[t2]\n\t"                                                             \
+    "v_sub_i32 %[t1], %[t1], %[t2] clamp\n\t"                                                           \
     "v_max_i32_e32 %[t1], %[t1], %[loy]\n\t"                                                            \
     "v_mad_i32_i24 %[idx], %[t1], %[nsty], %[idx]\n\t"                                                  \
     "v_fract_f32_e32 %[t0], %[sz]\n\t"                                                                  \
@@ -550,7 +552,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "s_and_b64 %[ta], %[ta], %[nbx]\n\t"                                                                \
     "v_cndmask_b32_e64 %[iz], %[iz], %[rz], %[ta]\n\t"                                                  \
     "v_cndmask_b32_e64 %[t2], 0, 1, %[ta]\n\t"                                                          \
-    "v_sub_u32_e32 %[t1], %[t1], %[t2]\n\t"                                                             \
+    "v_sub_i32 %[t1], %[t1], %[t2] clamp\n\t"                                                           \
     "v_max_i32_e32 %[t1], %[t1], %[loz]\n\t"                                                            \
     "v_mad_i32_i24 %[idx], %[t1], %[nstz], %[idx]\n\t"                                                  \
     "s_mov_b64 exec, %[jmp]\n\t"                                                                        \
