@@ -98,14 +98,28 @@ def jumps_and_solids(rng, dims):
 
 
 @pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
-@pytest.mark.parametrize("axis", [0, 2], ids=["x", "z"])
+@pytest.mark.parametrize("axis", [0, 1, 2, None], ids=["x", "y", "z", "all"])
 def test_long_directions(gpu, orc, dims, axis):
-    """One component of 2^20 to 2^60: most jumps end far outside the grid, many
-    beyond 2^31, where the cell saturates; the walk has to leave the grid there."""
-    rng = np.random.default_rng(40 + axis)
+    """One component of 2^20 to 2^60, or each of 2^-19 to 2^60: most jumps end far
+    outside the grid, many beyond 2^31, where the cell saturates; the walk has to
+    leave the grid there, one iteration later."""
+    rng = np.random.default_rng(40 if axis is None else 41 + axis)
     world = jumps_and_solids(rng, dims)
     n = 40000
     start = np.stack([rng.uniform(0.01, min(s, 48), n) for s in dims], 1)
     d = rng.choice([-1.0, 1.0], (n, 3)) * 2.0 ** rng.uniform(-8, 2, (n, 3))
-    d[:, axis] = rng.choice([-1.0, 1.0], n) * 2.0 ** rng.uniform(20, 60, n)
+    if axis is None:
+        d = rng.choice([-1.0, 1.0], (n, 3)) * 2.0 ** rng.uniform(-19, 60, (n, 3))
+    else:
+        d[:, axis] = rng.choice([-1.0, 1.0], n) * 2.0 ** rng.uniform(20, 60, n)
     compare(gpu, orc, world, dims, start, d, rng.integers(1, 200, n))
+
+
+def test_step_count_of_a_jump_beyond_two_to_the_31(gpu, orc):
+    """Two iterations: the step into the jump, then the one that leaves the grid
+    from beyond y = 2^31."""
+    dims = (24, 20, 40)
+    world = np.full(dims[0] * dims[1] * dims[2], -1, np.int32)
+    world[5 + dims[0] * (6 + dims[1] * 5)] = np.float32(-2.0).view(np.int32)
+    r = compare(gpu, orc, world, dims, [[5.5, 5.5, 5.5]], [[0.3, 2.0 ** 32, 0.3]], [200], 200)
+    assert r["steps"].tolist() == [2]

@@ -473,7 +473,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "v_cvt_flr_i32_f32_e32 %[t1], %[sy]\n\t"                                                            \
     "v_cmp_gt_f32_e32 vcc, %[lim], %[trav]\n\t"                                                         \
     "v_cmp_gt_f32_e64 %[ta], %[sy], %[tb]\n\t"                                                          \
-    "s_and_b64 exec, vcc, %[ta]\n\t" /* out of budget or grid, or above the solid top: a miss */        \
+    "s_and_b64 exec, vcc, %[ta]\n\t" /* out of budget, or above the solid top: a miss */                \
     "s_cbranch_execz 5f\n\t"                                                                            \
     "v_fract_f32_e32 %[ix], %[sx]\n\t"                                                                  \
     "v_fract_f32_e32 %[iy], %[sy]\n\t"                                                                  \
@@ -739,7 +739,9 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
     if constexpr (!std::is_same_v<IX, Idx64>) {
         Walk w;
         if (start_walk<IX, kHit>(g, px, py, pz, dx, dy, dz, w)) {
-            w.tb = dy > 0.0f ? -1.0f - (float)ytop : -__builtin_inff();
+            // s' > tb goes on; without a bound every s' does, whatever its size
+            const float bound = ytop == INT32_MAX ? -__builtin_inff() : -1.0f - (float)ytop;
+            w.tb = dy > 0.0f ? bound : -__builtin_inff();
             run_walk<kLanes>(IX{}, g.vox, lim, __ballot(0.0f < lim), w);
             auto flip = [](int32_t nst, float v) { return nst < 0 ? -v : v; };
             const bool bx = (w.ix < w.iy) & (w.ix < w.iz), by = (w.iy < w.ix) & (w.iy < w.iz);
