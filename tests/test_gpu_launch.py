@@ -106,11 +106,11 @@ def test_launch_shapes(gpu, orc, scene, size):
 
 
 def test_walks_begun_again_count_once(gpu):
-    """Where the wave's sum is counted (a plain draw beyond 16384 tiles), a walk
-    that run_walk gives up counts from then on in walk_generic; the persistent
-    launch counts each lane's.  A scene that has such walks (its sun rays leave
-    by the x-y edge), and others that reach the solid top at a whole y.  The
-    total is that of walk_generic taking every ray."""
+    """Where the wave's sum is counted (a plain draw beyond 16384 tiles, the
+    hardware-scheduled views), a walk that run_walk gives up counts from then on
+    in walk_generic; the persistent launch counts each lane's.  A scene that has
+    such walks (its sun rays leave by the x-y edge), and others that reach the
+    solid top at a whole y."""
     sc = gpu.make_scene("tiny", seed=1)
     size = (3840, 2160)
     f = sc.frame
@@ -118,12 +118,60 @@ def test_walks_begun_again_count_once(gpu):
     ctx = gpu.Context(sc.dims)
     ctx.upload(sc.world)
     ctx.build_depth_field()
+    out, lanes = views(gpu, ctx, f, size, 3)
+    assert lanes["dda_steps"] > 3e8
     ctx.stats(reset=True)
     t = gpu.Target(*size, depth=True, aux=False)
     ctx.draw(t, frame=f)
     st = ctx.stats(reset=True)
-    out, lanes = views(gpu, ctx, f, size, 3)
-    assert st["dda_steps"] == 171671802
     assert lanes["dda_steps"] == 2 * st["dda_steps"] and lanes["rays"] == 2 * st["rays"]
     assert np.array_equal(out[0]["rgb"], t.download()["rgb"])
+    hw = views(gpu, ctx, f, size, 0)[1]
+    assert hw["dda_steps"] == lanes["dda_steps"] and hw["rays"] == lanes["rays"]
+    ctx.close()
+
+
+def edge_scene(gpu, orc, dims, corner_words):
+    """Jumps near the edge x = y = 0 and a camera whose rays all descend in x and
+    y and leave there: many land with only x or only y below 0 and take their next
+    step along the other axis.  The one solid voxel lies above the camera, so no
+    ray takes the cutoff and the totals are the oracle's.  corner_words: some cells
+    hold the guard corner's bits (a NaN jump, which ends a walk)."""
+    rng = np.random.default_rng(5)
+    cells = dims[0] * dims[1] * dims[2]
+    world = np.full(cells, -1, np.int32)
+    jump = rng.random(cells) < 0.6
+    world[jump] = (-rng.uniform(0.5, 4.0, int(jump.sum())).astype(np.float32)).view(np.int32)
+    if corner_words:
+        world[rng.random(cells) < 0.05] = np.uint32(0xFFC00001).view(np.int32)
+    world[cells - 1] = 0x334455
+    f = gpu.frame_defaults(dims[0], 1024, 1024)
+    f.cam_pos[:] = [6.3, 7.1, 0.4 * dims[2]]
+    f.rotate_matrix[:] = gpu.camera_matrix(0.7, -0.5 * math.pi).tolist()
+    f.focal = 3.0
+    for vx in (-1.1, 1.1):  # beyond the widest picture below
+        for vy in (-1.0, 1.0):
+            d = orc.primary_dir(f, vx, vy)
+            assert d[0] < -0.2 and d[1] < -0.2, d
+    return world, f
+
+
+@pytest.mark.parametrize("corner_words", [False, True], ids=["edge", "words"])
+@pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
+def test_totals_of_walks_that_end_on_the_guard_corner(gpu, orc, dims, corner_words):
+    """Totals of the wave's sum where run_walk's last word is the guard corner's
+    and the shader's walk ends there too: the oracle's, and the persistent
+    launch's lane by lane."""
+    size = (1025, 1021)
+    world, f = edge_scene(gpu, orc, dims, corner_words)
+    f.aspect_ratio = size[0] / size[1]
+    r = orc.render(world, dims, f, *size)
+    assert r["rays"] == size[0] * size[1]  # every ray a miss
+    ctx = gpu.Context(dims)
+    ctx.upload(world)
+    ctx.stats(reset=True)
+    ctx.draw(gpu.Target(*size, depth=True, aux=False), frame=f)
+    assert ctx.stats(reset=True)["dda_steps"] == r["dda_steps"]
+    for chunk in (0, 3):
+        assert views(gpu, ctx, f, size, chunk)[1]["dda_steps"] == 2 * r["dda_steps"], chunk
     ctx.close()

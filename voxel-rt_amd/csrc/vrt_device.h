@@ -329,8 +329,9 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
             // the cutoff.
             if (!(trav < lim) | (cy > ytop)) break;
             if constexpr (kAgain) {
-                // run_walk's two ends: a tiny fraction at a jump, or the step
-                // after a jump to below both x = 0 and y = 0
+                // where this walk goes on and run_walk's does not: a tiny
+                // fraction at a jump, or the step after a jump to below both
+                // x = 0 and y = 0
                 const bool tiny = ((sx > 0.0f) & (sx < 0x1p-60f)) | ((sy > 0.0f) & (sy < 0x1p-60f)) |
                                   ((sz > 0.0f) & (sz < 0x1p-60f));
                 const bool edge = (sx < 0.0f) & (sy < 0.0f);
@@ -370,7 +371,11 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     h.index = result;
     h.axis = axis;
     h.step = axis == 0 ? stx : (axis == 1 ? sty : stz);
-    h.iters = kAgain ? iters - counted : iters;
+    // still `again`: this walk ended in the iteration that run_walk's ended in
+    // (a kGuardCorner that the shader's walk meets too: a cell beside the grid,
+    // reached along the other axis after a jump to below x = 0 or y = 0 alone,
+    // or a word of the caller's grid with the same bits)
+    h.iters = kAgain ? (again ? 0 : iters - counted) : iters;
 }
 
 // The same walk for 32-bit indices (IdxB, Idx32), where it is bound by VALU
@@ -415,7 +420,8 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // iteration.  The two differ only if x and y are both on their way out with
 // exactly equal intersects, for then the reference steps z.  Such a walk ends
 // on a guard cell with x < 0 and y < 0, which hold kGuardCorner: the ray is
-// then walked again by walk_generic.
+// then walked again by walk_generic.  (So are a few that end on one without
+// such a tie, with the same result.)
 //
 // The loop: a lane that hits drops out with its state as it was before the
 // step's update, so the axis, the intersect and the hit follow after the loop;
