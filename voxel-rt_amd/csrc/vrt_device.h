@@ -327,14 +327,19 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
             // a guard cell) ends the walk at the loop test (:83); nothing the
             // jump recomputes is read after that.  One branch for that and
             // the cutoff.
-            if (!(trav < lim) | (cy > ytop)) break;
+            if (!(trav < lim) | (cy > ytop)) {
+                // run_walk's last word, if in the caller's grid: both end here
+                if (kAgain && again & (v == kGuardCorner)) counted = iters;
+                break;
+            }
             if constexpr (kAgain) {
-                // where this walk goes on and run_walk's does not: a tiny
-                // fraction at a jump, or the step after a jump to below both
-                // x = 0 and y = 0
+                // where else run_walk ended: at a jump with a tiny fraction, or
+                // in the step after a jump to below x = 0 or y = 0 (`again`
+                // says that this step met the guard's corner: with both below
+                // 0, or along the other axis, when this walk ends there too)
                 const bool tiny = ((sx > 0.0f) & (sx < 0x1p-60f)) | ((sy > 0.0f) & (sy < 0x1p-60f)) |
                                   ((sz > 0.0f) & (sz < 0x1p-60f));
-                const bool edge = (sx < 0.0f) & (sy < 0.0f);
+                const bool edge = (sx < 0.0f) | (sy < 0.0f);
                 if (again & (tiny | edge)) {
                     counted = iters + (tiny ? 0 : 1);
                     again = false;
@@ -371,11 +376,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     h.index = result;
     h.axis = axis;
     h.step = axis == 0 ? stx : (axis == 1 ? sty : stz);
-    // still `again`: this walk ended in the iteration that run_walk's ended in
-    // (a kGuardCorner that the shader's walk meets too: a cell beside the grid,
-    // reached along the other axis after a jump to below x = 0 or y = 0 alone,
-    // or a word of the caller's grid with the same bits)
-    h.iters = kAgain ? (again ? 0 : iters - counted) : iters;
+    h.iters = kAgain ? iters - counted : iters;
 }
 
 // The same walk for 32-bit indices (IdxB, Idx32), where it is bound by VALU
@@ -397,7 +398,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // takes up the 1.
 //
 // Which rays: those whose direction components lie in [2^-19, 2^60] in
-// magnitude and whose start coordinates lie in [2^-20, 2^22] (cast_ray).  On an
+// magnitude and whose start coordinates lie in [2^-20, 2^22] (start_walk).  On an
 // ascending axis s then stays at least 2^-20, where the hardware's fraction is
 // the rounded difference; on a descending one s may fall below 0 only on its
 // way out of the grid (below).  Only the low end of a cell is clamped (lo:
