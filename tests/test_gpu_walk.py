@@ -7,6 +7,8 @@ indices."""
 import numpy as np
 import pytest
 
+import ray_orders
+
 pytestmark = pytest.mark.gpu
 
 GRIDS = [(24, 20, 40), (4096, 600, 2)]  # byte offsets; 4 X Y >= 2^23: word indices
@@ -19,7 +21,7 @@ def compare(gpu, orc, world, dims, start, d, dist, budget=256):
     ctx.upload(world)
     r = orc.cast_rays(world, dims, start, d, dist, budget)
     for steps in (True, False):
-        g = ctx.cast_rays(start, d, dist, budget, steps=steps)
+        g = ray_orders.cast_rays(ctx, start, d, dist, budget, steps=steps)
         for k in ("hit", "face", "steps") if steps else ("hit", "face"):
             bad = np.nonzero(g[k] != r[k])[0]
             assert bad.size == 0, "%s differs for %d rays, first start %s dir %s: %s, oracle %s" % (
