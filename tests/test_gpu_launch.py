@@ -1,4 +1,4 @@
-"""Launch shapes of the render kernels (wave_item, split_tile, lane_counts):
+"""Launch shapes of the render kernels (wave_item, split_tile, draw_form):
 tile counts around a workgroup, around a round of workgroups over the XCDs and
 on either side of 16384 tiles, one wave a workgroup (byte offsets) and four
 (word indices), as a plain draw, a hardware-scheduled launch of views and a
@@ -175,3 +175,46 @@ def test_totals_of_walks_that_end_on_the_guard_corner(gpu, orc, dims, corner_wor
     for chunk in (0, 3):
         assert views(gpu, ctx, f, size, chunk)[1]["dda_steps"] == 2 * r["dda_steps"], chunk
     ctx.close()
+
+
+@pytest.fixture(scope="module")
+def large(gpu):
+    """A copy over 3.25 GiB that is at least 1400 long on x and z and 256 high."""
+    dims = (1408, 256, 2400)
+    p = gpu.world_params(dims, 3, caves=2000)
+    ctx = gpu.Context(dims)
+    ctx.generate(p)
+    ctx.build_depth_field()
+    yield dims, p, ctx, ctx.download()
+    ctx.close()
+
+
+@pytest.mark.parametrize("size", [(3, 8), (33, 8), (72, 56), (257, 131)], ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("dist", [1399, 1400, 4000])
+def test_far_views_in_four_wave_groups(gpu, orc, large, dist, size):
+    """draw_form on either side of its render distance: a depth view and a step
+    map, as a plain draw, hardware-scheduled and persistent views."""
+    dims, p, ctx, words = large
+    f = gpu.frame_defaults(dims[0], *size)
+    x, z = dims[0] // 2, 200
+    f.cam_pos[:] = [x + 0.3, gpu.surface(p, x, z) + 12.6, z + 0.4]
+    f.rotate_matrix[:] = gpu.camera_matrix(0.05, 0.1).tolist()
+    f.aspect_ratio = size[0] / size[1]
+    f.render_dist = dist
+    for depth_view in (1, 0):
+        f.view_depth_field = depth_view
+        t = gpu.Target(*size, depth=True, aux=True)
+        ctx.stats(reset=True)
+        ctx.draw(t, frame=f)
+        st = ctx.stats(reset=True)
+        g, r = t.download(), orc.render(words, dims, f, *size)
+        for k in ("hit", "face", "steps", "shadow_eval", "shadow_occ"):
+            assert np.array_equal(g[k], r[k]), (depth_view, k)
+        assert int(np.abs(g["rgb"].astype(np.int16) - r["rgb"].astype(np.int16)).max()) <= RGB_TOL
+        assert st["rays"] == r["rays"] and st["pixels"] == size[0] * size[1]
+        if depth_view:  # no ray takes the cutoff
+            assert st["dda_steps"] == r["dda_steps"]
+            for chunk in (0, 3):
+                out, s = views(gpu, ctx, f, size, chunk)
+                assert all(np.array_equal(o["rgb"], g["rgb"]) for o in out), chunk
+                assert s["dda_steps"] == 2 * st["dda_steps"] and s["pixels"] == 2 * st["pixels"], chunk

@@ -165,7 +165,8 @@ int vrt_batch_create(vrt_ctx* ctx, const vrt_view* views, int32_t n, const vrt_b
     int rc = cfg.chunk_tiles ? launch_queue_reset(b->queue, b->capture) : VRT_OK;
     if (!rc)
         rc = launch_render_batch(render_grid(ctx), b->views_dev, (int32_t)b->views.size(), b->total_tiles, cfg,
-                                 lane_counts(render_grid(ctx), b->views), b->workgroups, b->queue, ctx->counters, b->parts, b->capture);
+                                 draw_form(render_grid(ctx), b->views), b->workgroups, b->queue, ctx->counters,
+                                 b->parts, b->capture);
     if (!rc && b->parts) rc = launch_fold_parts(b->parts, b->items, ctx->counters, b->capture);
     e = hipStreamEndCapture(b->capture, &b->graph);
     if (rc) return bail(rc);

@@ -153,17 +153,27 @@ int launch_fold_parts(const unsigned long long* parts, int64_t n, unsigned long 
 int launch_cast_rays(const GridDesc& g, int64_t n, const float* start, const float* dir,
                      const int32_t* dist, int32_t render_dist, int64_t* hit, float* hit_pos,
                      uint8_t* face, uint32_t* steps, hipStream_t s);
+// How a launch's waves count (lanes: each lane its iterations) and are grouped
+// (far: four a workgroup); for several views, what any of them needs.
+struct DrawForm {
+    bool lanes = false, far = false;
+    DrawForm& operator|=(const DrawForm& o) {
+        lanes |= o.lanes;
+        far |= o.far;
+        return *this;
+    }
+};
+DrawForm draw_form(const GridDesc& g, const FrameDesc& f);
 // parts (chunk_tiles 0 only; nullptr: atomics): one entry per 64-pixel pass
 // (batch_items), added into the counters by launch_fold_parts afterwards.
-bool lane_counts(const GridDesc& g, const FrameDesc& f);  // for `lanes`: true if it is for any view
 int launch_render_batch(const GridDesc& g, const ViewDesc* views_dev, int32_t n_views,
-                        int64_t total_tiles, const vrt_batch_config& cfg, bool lanes, int32_t n_workgroups,
+                        int64_t total_tiles, const vrt_batch_config& cfg, DrawForm form, int32_t n_workgroups,
                         unsigned int* queue, unsigned long long* counters, unsigned long long* parts,
                         hipStream_t s);
-inline bool lane_counts(const GridDesc& g, const std::vector<ViewDesc>& views) {
-    bool any = false;
-    for (const ViewDesc& v : views) any |= lane_counts(g, v.frame);
-    return any;
+inline DrawForm draw_form(const GridDesc& g, const std::vector<ViewDesc>& views) {
+    DrawForm form;
+    for (const ViewDesc& v : views) form |= draw_form(g, v.frame);
+    return form;
 }
 // Entries a hardware-scheduled multi-view launch writes into `parts`, or -1
 // when its counts must go by atomics (a view's render_lim too large for the

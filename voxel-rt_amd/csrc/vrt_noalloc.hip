@@ -100,14 +100,14 @@ int vrt_draw_views_noalloc(vrt_ctx* ctx, const vrt_view* views, int32_t n, const
     }
     // descriptors built four at a time and passed by value to a copy kernel
     int64_t total_tiles = 0;
-    bool lanes = false;
+    DrawForm form;
     for (int32_t i = 0; i < n; i += kPutPerLaunch) {
         const int32_t k = n - i < kPutPerLaunch ? n - i : kPutPerLaunch;
         ViewPack pack{};
         for (int32_t j = 0; j < k; j++) {
             if (int rc = make_view_desc(views[order[i + j]], cfg, total_tiles, pack.v[j])) return rc;
             total_tiles += pack.v[j].tiles;
-            lanes |= lane_counts(render_grid(ctx), pack.v[j].frame);
+            form |= draw_form(render_grid(ctx), pack.v[j].frame);
         }
         if (total_tiles > kMaxBatchTiles) return fail(VRT_ERR_INVALID, "too many tiles in one call");
         hipLaunchKernelGGL(k_put_views, dim3(1), dim3(256), 0, ctx->stream, views_dev + i, k, pack);
@@ -117,7 +117,7 @@ int vrt_draw_views_noalloc(vrt_ctx* ctx, const vrt_view* views, int32_t n, const
     if (int rc = persistent_workgroups(ctx, cfg, total_tiles, &wgs)) return rc;
     if (cfg.chunk_tiles)
         if (int rc = launch_queue_reset(queue, ctx->stream)) return rc;  // a kernel, not a memset
-    if (int rc = launch_render_batch(render_grid(ctx), views_dev, n, total_tiles, cfg, lanes, wgs, queue,
+    if (int rc = launch_render_batch(render_grid(ctx), views_dev, n, total_tiles, cfg, form, wgs, queue,
                                      ctx->counters, nullptr, ctx->stream))
         return rc;
     ctx->draws += (uint64_t)n;

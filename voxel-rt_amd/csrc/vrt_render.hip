@@ -26,31 +26,31 @@ constexpr int kXcds = 8;
 // Waves per workgroup of the hardware-scheduled kernels.  A 4-wave workgroup
 // starts only when one CU has a slot free on each of its SIMDs, so slots stand
 // empty meanwhile; one-wave workgroups fill them at once.  But the four
-// adjacent tiles of a 4-wave workgroup share a CU's L1, which is worth more
-// where walks spread over a render copy beyond 4 GiB (Idx32, Idx64).  Four waves
-// against one: 1080p in a 256 MiB grid 107.8 and 102.3 us, 1366x768 with all
-// maps 74.3 and 67.9, 3840x2160 in a 1 GiB grid 326 and 319, 320x180 30.0 and
-// 28.8; 3840x2160 in the 8 GiB grid 340 and 358, its depth view 1.39 and 1.95 ms.
+// adjacent tiles of a 4-wave workgroup share a CU's L1 (17.7 M reads from beyond
+// it for 27.7 M, depth view at 1080p in a 3.7 GiB copy), which is worth more
+// where walks spread over a render copy beyond 4 GiB (Idx32, Idx64) or far over
+// one that is nearly as large (draw_form).  Four waves against one: 1080p in a
+// 256 MiB grid 107.8 and 102.3 us, 1366x768 with all maps 74.3 and 67.9,
+// 3840x2160 in a 1 GiB grid 326 and 319, 320x180 30.0 and 28.8; 3840x2160 in the
+// 8 GiB grid 340 and 358, its depth view 1.39 and 1.95 ms.
 // (Two waves lie between; eight are 18% slower at 1080p.)
+constexpr int kGroupWaves = 4;
 template <typename IX>
-constexpr int kWavesPerGroup = std::is_same_v<IX, dev::IdxB> ? 1 : 4;
+constexpr int kNearGroupWaves = std::is_same_v<IX, dev::IdxB> ? 1 : kGroupWaves;
 
 // The tile or pass that a wave takes.  Workgroups go to the XCDs round-robin;
 // runs of four items stay on one XCD and its L2 (one-wave workgroups b, b + 8,
 // b + 16, b + 24 of each 32; without that 1366x768 took 72.2 us), so every XCD
 // still gets an even share of sky, horizon and terrain tiles.  (A contiguous
 // band of rows per XCD had the better hit rate but unequal loads, 29% slower.)
-template <typename IX>
+template <int kGroup>
 __device__ __forceinline__ uint32_t wave_item() {
     const uint32_t b = blockIdx.x;
-    if constexpr (kWavesPerGroup<IX> == 1) return ((b / 32) * kXcds + b % kXcds) * 4 + (b / kXcds) % 4;
-    return b * kWavesPerGroup<IX> + (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)(threadIdx.x >> 6));
+    if constexpr (kGroup == 1) return ((b / 32) * kXcds + b % kXcds) * 4 + (b / kXcds) % 4;
+    return b * kGroup + (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)(threadIdx.x >> 6));
 }
-// Workgroups for n items.
-template <typename IX>
-int64_t groups_for(int64_t n) {
-    return kWavesPerGroup<IX> == 1 ? (n + 31) / 32 * 32 : (n + kWavesPerGroup<IX> - 1) / kWavesPerGroup<IX>;
-}
+// Workgroups of `group` waves for n items.
+int64_t groups_for(int group, int64_t n) { return group == 1 ? (n + 31) / 32 * 32 : (n + group - 1) / group; }
 constexpr int kQueueStride = 32;  // queue counters 128 bytes apart
 
 // n / d and n % d for a wave-uniform n, on the scalar unit, from rcp =
@@ -107,14 +107,14 @@ __device__ __forceinline__ void flush_counters_tile(unsigned long long* counters
 // waves_per_eu(8, 8): without it the build ran at 7 resident waves per SIMD
 // (peak measured with per-wave timestamps: 7168 waves on 1024 SIMDs); with it,
 // 8 (a few registers of the rare IEEE-division path spill), 4% faster.
-template <typename IX, bool kLanes>
-__global__ void __launch_bounds__(kWave * kWavesPerGroup<IX>) __attribute__((amdgpu_waves_per_eu(8, 8)))
+template <typename IX, bool kLanes, int kGroup>
+__global__ void __launch_bounds__(kWave * kGroup) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_render_plain(GridDesc g, FrameDesc F, vrt_target t, unsigned long long* counters, unsigned long long* parts) {
     const int32_t top = g.top ? *g.top : INT32_MAX;
     const int32_t tiles_x = (t.width + 7) >> 3;
     const int32_t tiles_y = (t.height + 7) >> 3;
     // the wave's tile is uniform: the tile arithmetic runs on the scalar unit
-    const int32_t tile = (int32_t)wave_item<IX>();
+    const int32_t tile = (int32_t)wave_item<kGroup>();
     const int32_t lane = threadIdx.x & 63;
     uint32_t rays = 0, iters = 0, pixels = 0;
     if (tile < tiles_x * tiles_y) {
@@ -226,14 +226,14 @@ __device__ __forceinline__ void shade_view_tile(const GridDesc& g, const ViewDes
 // tile shape within 64 VGPRs without spilling.  The dispatcher hands out
 // workgroups in order as slots free up, so the views' tiles are balanced over
 // the device without any queue.
-template <typename IX, int TW, int TH, bool kLanes>
-__global__ void __launch_bounds__(kWave * kWavesPerGroup<IX>) __attribute__((amdgpu_waves_per_eu(8, 8)))
+template <typename IX, int TW, int TH, bool kLanes, int kGroup>
+__global__ void __launch_bounds__(kWave * kGroup) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_render_views(GridDesc g, const ViewDesc* __restrict__ views, int32_t n_views, int64_t total_tiles,
                unsigned long long* counters, unsigned long long* parts) {
     constexpr int32_t kPasses = TW * TH / kWave;
     const int32_t top = g.top ? *g.top : INT32_MAX;
     const int32_t lane = threadIdx.x & 63;
-    const int64_t item = (int64_t)wave_item<IX>();
+    const int64_t item = (int64_t)wave_item<kGroup>();
     uint32_t rays = 0, iters = 0, pixels = 0;
     if (item < total_tiles * kPasses)
         shade_view_tile<IX, TW, TH, kLanes>(g, views, n_views, item / kPasses, (int32_t)(item % kPasses), 1, lane, top, rays,
@@ -338,13 +338,24 @@ void with_index(const GridDesc& g, F&& f) {
 
 }  // namespace
 
-// Whether a frame's iterations have to be counted lane by lane (one VALU
-// instruction an iteration more than the wave's sum, which takes two scalar
-// ones): a step map or the depth view shows them, and the wave's sum has to fit
-// 32 bits.  (primary_cutoff is 0 with a step map, in the depth view, and with the
-// cutoff switched off, where totals are compared with the reference's.)
-bool lane_counts(const GridDesc& g, const FrameDesc& f) {
-    return f.primary_cutoff == 0 || g.top == nullptr || !(f.render_lim < kTileSum32Lim);
+// Lane by lane: one VALU instruction an iteration more than the wave's sum, which
+// takes two scalar ones; needed where a step map or the depth view shows the
+// counts, and where the wave's sum could exceed 32 bits.  (primary_cutoff is 0
+// with a step map, in the depth view, and with the cutoff switched off, where
+// totals are compared with the reference's.)
+//
+// Far: walks that no cutoff ends, in a copy over 3.25 GiB in which they can run
+// 1400 cells along x and z and 256 up.  Depth view at 3840x2160, one wave a group
+// and four: 1600x400x1600 (3.9 GiB) 1267 and 1065 us at the worst camera,
+// 2048x256x1900 1130 and 1025; over four cameras at two sizes one wave takes 2 to
+// 3% more there, 2% less in 2048x256x1490 (3.0 GiB), 4% less in 2400x170x2400 and
+// 1024x256x3750, and 1 to 3% less in any at a render distance of 384.
+DrawForm draw_form(const GridDesc& g, const FrameDesc& f) {
+    DrawForm d;
+    d.lanes = f.primary_cutoff == 0 || g.top == nullptr || !(f.render_lim < kTileSum32Lim);
+    const float run = std::min((float)std::min(g.X, g.Z), f.render_lim);
+    d.far = d.lanes && g.count > (13ull << 26) && g.Y >= 256 && run >= 1400.0f;
+    return d;
 }
 
 int launch_render_plain(const GridDesc& g, const FrameDesc& f, const vrt_target& t, unsigned long long* counters,
@@ -357,10 +368,15 @@ int launch_render_plain(const GridDesc& g, const FrameDesc& f, const vrt_target&
         // views in one launch 5.76 -> 5.68 ms, 3840x2160 346 -> 341 us), not
         // where a frame has less than about two tiles for each of the 8,192
         // wave slots and waits for its longest walk (320x180: 30.0 -> 30.3 us).
-        const bool lanes = lane_counts(g, f) || tiles <= 16384;
-        auto* kernel = lanes ? k_render_plain<decltype(ix), true> : k_render_plain<decltype(ix), false>;
-        hipLaunchKernelGGL(kernel, dim3((uint32_t)groups_for<decltype(ix)>(tiles)),
-                           dim3(kWave * kWavesPerGroup<decltype(ix)>), 0, s, g, f, t, counters, parts);
+        using IX = decltype(ix);
+        constexpr int kNear = kNearGroupWaves<IX>;
+        const DrawForm form = draw_form(g, f);
+        auto* kernel = form.far                        ? k_render_plain<IX, true, kGroupWaves>
+                       : form.lanes || tiles <= 16384 ? k_render_plain<IX, true, kNear>
+                                                       : k_render_plain<IX, false, kNear>;
+        const int group = form.far ? kGroupWaves : kNear;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)groups_for(group, tiles)), dim3(kWave * group), 0, s, g, f, t,
+                           counters, parts);
     });
     VRT_HIP(hipGetLastError());
     return VRT_OK;
@@ -410,7 +426,7 @@ int batch_occupancy(const vrt_batch_config& cfg, int32_t* waves_per_cu) {
 }
 
 int launch_render_batch(const GridDesc& g, const ViewDesc* views_dev, int32_t n_views, int64_t total_tiles,
-                        const vrt_batch_config& cfg, bool lanes, int32_t n_workgroups, unsigned int* queue,
+                        const vrt_batch_config& cfg, DrawForm form, int32_t n_workgroups, unsigned int* queue,
                         unsigned long long* counters, unsigned long long* parts, hipStream_t s) {
     if (parts && cfg.chunk_tiles != 0) return fail(VRT_ERR_INVALID, "partial counts need the hardware-scheduled kernel");
     if (cfg.chunk_tiles == 0) {
@@ -419,12 +435,14 @@ int launch_render_batch(const GridDesc& g, const ViewDesc* views_dev, int32_t n_
         if (items > 0x7fffffe0) return fail(VRT_ERR_INVALID, "too many tiles in one batch");
         if (int rc = with_shape(cfg.tile_w, cfg.tile_h, [&](auto tw, auto th) {
                 with_index(g, [&](auto ix) {
-                    constexpr int TW = decltype(tw)::value, TH = decltype(th)::value;
-                    auto* kernel =
-                        lanes ? k_render_views<decltype(ix), TW, TH, true> : k_render_views<decltype(ix), TW, TH, false>;
-                    const int64_t wgs = groups_for<decltype(ix)>(items);
-                    hipLaunchKernelGGL(kernel, dim3((uint32_t)wgs), dim3(kWave * kWavesPerGroup<decltype(ix)>), 0, s,
-                                       g, views_dev, n_views, total_tiles, counters, parts);
+                    using IX = decltype(ix);
+                    constexpr int TW = decltype(tw)::value, TH = decltype(th)::value, kNear = kNearGroupWaves<IX>;
+                    auto* kernel = form.far     ? k_render_views<IX, TW, TH, true, kGroupWaves>
+                                   : form.lanes ? k_render_views<IX, TW, TH, true, kNear>
+                                                : k_render_views<IX, TW, TH, false, kNear>;
+                    const int group = form.far ? kGroupWaves : kNear;
+                    hipLaunchKernelGGL(kernel, dim3((uint32_t)groups_for(group, items)), dim3(kWave * group), 0, s, g,
+                                       views_dev, n_views, total_tiles, counters, parts);
                 });
             }))
             return rc;

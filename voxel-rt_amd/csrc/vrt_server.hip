@@ -289,7 +289,7 @@ int launch_slot(vrt_server* s, Slot& sl, std::vector<uint64_t>& ids) {
     g.vox = s->copy[sl.copy].vox;
     const int64_t items = batch_items(descs, total, cfg);
     unsigned long long* parts = items > 0 && items <= kSlotParts ? sl.parts : nullptr;
-    if (int rc = launch_render_batch(g, sl.views_dev, (int32_t)descs.size(), total, cfg, lane_counts(g, descs), wgs,
+    if (int rc = launch_render_batch(g, sl.views_dev, (int32_t)descs.size(), total, cfg, draw_form(g, descs), wgs,
                                      sl.queue, c->counters, parts, sl.stream))
         return rc;
     if (parts)
