@@ -306,6 +306,8 @@ int remove_sphere_on(vrt_ctx* c, const GridDesc& render, int32_t cx, int32_t cy,
                      hipStream_t s) {
     const int32_t R = std::max(0, radius + (VRT_DEPTH_FIELD_RADIUS >> 1));
     const int64_t M = sphere_reach(radius);
+    // nothing carved, nothing repaired: the copy alone (4 us, k_edit_box 10)
+    if (R == 0 && radius <= 0) return render.vox ? remove_sphere_refresh_into(c, render, cx, cy, cz, radius, s) : VRT_OK;
     return launch_edit_box(c->grid, render, c->words, (int64_t)cx - M, (int64_t)cy - M, (int64_t)cz - M,
                            (int64_t)cx + M, (int64_t)cy + M, (int64_t)cz + M, cx, cy, cz, R, radius, s);
 }
