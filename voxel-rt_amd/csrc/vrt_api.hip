@@ -7,7 +7,6 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
-#include <numeric>
 #include <string>
 
 #include "vrt_internal.h"
@@ -57,18 +56,6 @@ std::vector<TableEntry> reference_table() {
     return t;
 }
 }  // namespace
-
-std::vector<float> depth_table_dist() {
-    std::vector<float> out;
-    for (auto& e : reference_table()) out.push_back(e.dist);
-    return out;
-}
-
-std::vector<int32_t> depth_table_offsets() {
-    std::vector<int32_t> out;
-    for (auto& e : reference_table()) out.insert(out.end(), {e.x, e.y, e.z});
-    return out;
-}
 
 // Largest float t with sqrtf(t) <= r (IEEE sqrt, correctly rounded like the
 // device's); NaN for NaN r, -inf when no t qualifies (r < 0).

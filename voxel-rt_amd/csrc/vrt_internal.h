@@ -225,8 +225,6 @@ int launch_world_generate(const GridDesc& g, const vrt_world_params& p, const in
                           int32_t bins_x, int32_t bins_z, hipStream_t s);
 
 // ---- host helpers
-std::vector<float> depth_table_dist();              // reference order
-std::vector<int32_t> depth_table_offsets();         // reference order, xyz triples
 double now_seconds();
 
 // World generator pieces shared by the host and device generators.
@@ -304,8 +302,8 @@ int check_batch_config(const vrt_batch_config& c);
 // first_tile; checks the frame and target.
 struct ViewDesc;
 int make_view_desc(const vrt_view& v, const vrt_batch_config& cfg, int64_t first_tile, ViewDesc& d);
-// Workgroups of a multi-view launch: one per four tiles when the hardware
-// schedules (chunk_tiles 0), else persistent workgroups from occupancy.
+// Persistent workgroups of a multi-view launch, from occupancy; 0 when the
+// hardware schedules (chunk_tiles 0), where the launch counts its own.
 int persistent_workgroups(vrt_ctx* c, const vrt_batch_config& cfg, int64_t total_tiles, int32_t* out);
 int check_target(const vrt_target& t);
 }  // namespace vrt
