@@ -745,15 +745,17 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
     h.iters = 0;
     if constexpr (!std::is_same_v<IX, Idx64>) {
         Walk w;
-        // One lane that run_walk does not take sends the wave to walk_generic:
-        // two walks one after the other cost the wave the time of both.  Such
-        // lanes are few (a pixel in 700 along the horizon, where a component is
-        // below 2^-19), but their waves are a frame's longest.  Depth view,
-        // 1920x1080 in a 512x512x3700 grid: 400 us, each lane by its own walk 511;
-        // shaded frames alike.  (Taking such rays too, by a test of |d + 1e-6|: the
-        // same there, 16 views in one launch 1% slower.)
+        // One lane that run_walk does not take sends the wave to walk_generic
+        // where the lanes count (a depth view or step map, whose walks are
+        // long): two walks one after the other cost the wave the time of both.
+        // Such lanes are few (a pixel in 700 along the horizon, where a component
+        // is below 2^-19), but their waves are a frame's longest.  Depth view,
+        // 1920x1080 in a 512x512x3700 grid: 400 us, each lane by its own walk
+        // 511.  (In shaded frames no gain, and at 3840x2160 1% more for the test.
+        // Taking such rays too, by a test of |d + 1e-6|: the same for the depth
+        // view, 16 views in one launch 1% slower.)
         const bool fast = start_walk<IX, kHit>(g, px, py, pz, dx, dy, dz, w);
-        if (__ballot(!fast) == 0) {
+        if (kLanes ? __ballot(!fast) == 0 : fast) {
             // s' > tb goes on; without a bound every s' does, whatever its size
             const float bound = ytop == INT32_MAX ? -__builtin_inff() : -1.0f - (float)ytop;
             w.tb = dy > 0.0f ? bound : -__builtin_inff();
