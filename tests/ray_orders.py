@@ -6,7 +6,7 @@ import numpy as np
 
 def run_walk_takes(start, d):
     with np.errstate(invalid="ignore"):
-        return ((start >= 2.0 ** -20) & (start <= 2.0 ** 22) & (abs(d) >= 2.0 ** -19) & (abs(d) <= 2.0 ** 60)).all(1)
+        return ((start >= 2.0 ** -20) & (start <= 2.0 ** 22) & (abs(d) >= 2.0 ** -19) & (abs(d) <= 2.0 ** 6)).all(1)
 
 
 def cast_rays(ctx, start, d, dist, budget, steps=True):

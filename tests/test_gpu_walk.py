@@ -104,7 +104,8 @@ def jumps_and_solids(rng, dims):
 def test_long_directions(gpu, orc, dims, axis):
     """One component of 2^20 to 2^60, or each of 2^-19 to 2^60: most jumps end far
     outside the grid, many beyond 2^31, where the cell saturates; the walk has to
-    leave the grid there, one iteration later."""
+    leave the grid there, one iteration later.  (run_walk takes none of the first,
+    and of the others those up to 2^6.)"""
     rng = np.random.default_rng(40 if axis is None else 41 + axis)
     world = jumps_and_solids(rng, dims)
     n = 40000
@@ -115,6 +116,23 @@ def test_long_directions(gpu, orc, dims, axis):
     else:
         d[:, axis] = rng.choice([-1.0, 1.0], n) * 2.0 ** rng.uniform(20, 60, n)
     compare(gpu, orc, world, dims, start, d, rng.integers(1, 200, n))
+
+
+@pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
+def test_longest_jumps_that_run_walk_takes(gpu, orc, dims):
+    """Components up to 2^6, jumps and budgets up to 2^24: positions up to 2^30,
+    short of where a cell saturates."""
+    rng = np.random.default_rng(46)
+    cells = dims[0] * dims[1] * dims[2]
+    world = np.full(cells, -1, np.int32)
+    jump = rng.random(cells) < 0.3
+    world[jump] = (-(2.0 ** rng.uniform(0, 24, int(jump.sum()))).astype(np.float32)).view(np.int32)
+    solid = rng.random(cells) < 0.04
+    world[solid] = rng.integers(0, 1 << 24, int(solid.sum()))
+    n = 40000
+    start = np.stack([rng.uniform(0.01, min(s, 48), n) for s in dims], 1)
+    d = rng.choice([-1.0, 1.0], (n, 3)) * np.minimum(2.0 ** rng.uniform(-19, 8, (n, 3)), 2.0 ** 6)
+    compare(gpu, orc, world, dims, start, d, np.full(n, 1 << 24), 1 << 24)
 
 
 def test_step_count_of_a_jump_beyond_two_to_the_31(gpu, orc):

@@ -397,13 +397,16 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // word index is base + sum of floor(s') times the step's negated stride; base
 // takes up the 1.
 //
-// Which rays: those whose direction components lie in [2^-19, 2^60] in
+// Which rays: those whose direction components lie in [2^-19, 2^6] in
 // magnitude and whose start coordinates lie in [2^-20, 2^22] (start_walk).  On an
 // ascending axis s then stays at least 2^-20, where the hardware's fraction is
 // the rounded difference; on a descending one s may fall below 0 only on its
 // way out of the grid (below).  Only the low end of a cell is clamped (lo:
 // clamp_cell's -2 or n + 1, mirrored): a ray jumps from inside the grid,
-// downward on every axis.
+// downward on every axis.  And |s'| stays below 2^31, where a cell would
+// saturate and no bound on y (INT32_MAX) would become one: a jump goes less than
+// 2^24 (the budget's limit) times 2^6 beyond a segment's steps, whose cells lie
+// in a grid of less than 2^23 a side.
 //
 // After a jump a fraction may be below 2^-60, where the quotient's three
 // instructions are not exact (label 6).  Where s is whole it is 0, and the
@@ -411,9 +414,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // ascending one (the quotient RN(1/|d|)), whose cell is then one lower than
 // floor(s') says.  A tiny fraction that is not 0 takes the ray to
 // walk_generic.  (s beyond 2^23 is whole, and outside any grid with 32-bit
-// indices.  Beyond 2^31, where only directions longer than a unit vector reach,
-// floor(s') is INT32_MIN and the subtraction saturates: wrapped round to
-// INT32_MAX it would pass the clamp, and its low 24 bits are cell 0.)
+// indices.)
 //
 // Leaving through a low face.  For -1 < s < 0 the reference's cell is 0, with
 // a negative intersect that its next step takes at once, out of the grid; here
@@ -527,7 +528,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "s_and_b64 %[ta], %[ta], %[nbx]\n\t"                                                                \
     "v_cndmask_b32_e64 %[ix], %[ix], %[rx], %[ta]\n\t"                                                  \
     "v_cndmask_b32_e64 %[t2], 0, 1, %[ta]\n\t"                                                          \
-    "v_sub_i32 %[t1], %[t1], %[t2] clamp\n\t"                                                           \
+    "v_sub_u32_e32 %[t1], %[t1], %[t2]\n\t"                                                             \
     "v_max_i32_e32 %[t1], %[t1], %[lox]\n\t"                                                            \
     "v_mad_i32_i24 %[idx], %[t1], %[nstx], %[idx]\n\t"                                                  \
     "v_fract_f32_e32 %[t0], %[sy]\n\t"                                                                  \
@@ -543,7 +544,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "s_and_b64 %[ta], %[ta], %[nbx]\n\t"                                                                \
     "v_cndmask_b32_e64 %[iy], %[iy], %[ry], %[ta]\n\t"                                                  \
     "v_cndmask_b32_e64 %[t2], 0, 1, %[ta]\n\t"                                                          \
-    "v_sub_i32 %[t1], %[t1], %[t2] clamp\n\t"                                                           \
+    "v_sub_u32_e32 %[t1], %[t1], %[t2]\n\t"                                                             \
     "v_max_i32_e32 %[t1], %[t1], %[loy]\n\t"                                                            \
     "v_mad_i32_i24 %[idx], %[t1], %[nsty], %[idx]\n\t"                                                  \
     "v_fract_f32_e32 %[t0], %[sz]\n\t"                                                                  \
@@ -559,7 +560,7 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
     "s_and_b64 %[ta], %[ta], %[nbx]\n\t"                                                                \
     "v_cndmask_b32_e64 %[iz], %[iz], %[rz], %[ta]\n\t"                                                  \
     "v_cndmask_b32_e64 %[t2], 0, 1, %[ta]\n\t"                                                          \
-    "v_sub_i32 %[t1], %[t1], %[t2] clamp\n\t"                                                           \
+    "v_sub_u32_e32 %[t1], %[t1], %[t2]\n\t"                                                             \
     "v_max_i32_e32 %[t1], %[t1], %[loz]\n\t"                                                            \
     "v_mad_i32_i24 %[idx], %[t1], %[nstz], %[idx]\n\t"                                                  \
     "s_mov_b64 exec, %[jmp]\n\t"                                                                        \
@@ -666,7 +667,7 @@ __device__ __forceinline__ bool start_walk(const GridDesc& g, float px, float py
     // NaN; the comparisons of s (NaN where d is) or the sum do not.
     const float lo = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
     const float hi = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz));
-    bool fast = (lo >= 0x1p-19f) & (hi <= 0x1p60f);
+    bool fast = (lo >= 0x1p-19f) & (hi <= 0x1p6f);
     if constexpr (kHit) {
         w.ix = __builtin_amdgcn_fractf(w.sx);
         w.iy = __builtin_amdgcn_fractf(w.sy);
@@ -756,9 +757,7 @@ __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, 
         // view, 16 views in one launch 1% slower.)
         const bool fast = start_walk<IX, kHit>(g, px, py, pz, dx, dy, dz, w);
         if (kLanes ? __ballot(!fast) == 0 : fast) {
-            // s' > tb goes on; without a bound every s' does, whatever its size
-            const float bound = ytop == INT32_MAX ? -__builtin_inff() : -1.0f - (float)ytop;
-            w.tb = dy > 0.0f ? bound : -__builtin_inff();
+            w.tb = dy > 0.0f ? -1.0f - (float)ytop : -__builtin_inff();
             run_walk<kLanes>(IX{}, g.vox, lim, __ballot(0.0f < lim), w);
             auto flip = [](int32_t nst, float v) { return nst < 0 ? -v : v; };
             const bool bx = (w.ix < w.iy) & (w.ix < w.iz), by = (w.iy < w.ix) & (w.iy < w.iz);
