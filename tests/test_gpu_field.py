@@ -6,8 +6,6 @@ is read back through rays."""
 import numpy as np
 import pytest
 
-import ray_orders
-
 pytestmark = pytest.mark.gpu
 
 
@@ -27,7 +25,7 @@ def check_rays(gpu, orc, ctx, words, dims, rng, n=4000):
     start = np.stack([rng.uniform(-1.5, d + 1.5, n) for d in dims], 1).astype(np.float32)
     d = rng.normal(size=(n, 3)).astype(np.float32)
     dist = rng.integers(1, 200, n).astype(np.int32)
-    g = ray_orders.cast_rays(ctx, start, d, dist, 256)
+    g = ctx.cast_rays(start, d, dist, 256)
     r = orc.cast_rays(words, dims, start, d, dist, 256)
     for k in ("hit", "face", "steps"):
         assert np.array_equal(g[k], r[k]), "%s differs for %d rays" % (k, int((g[k] != r[k]).sum()))
@@ -137,7 +135,7 @@ def test_region_upload_in_pieces(gpu, orc, lo, size):
     d = rng.normal(size=(n, 3)).astype(np.float32)
     d[:, 1] = np.abs(d[:, 1])
     dist = np.full(n, 300, np.int32)
-    g, r = ray_orders.cast_rays(ctx, start, d, dist, 384, steps=False), orc.cast_rays(ref, dims, start, d, dist, 384)
+    g, r = ctx.cast_rays(start, d, dist, 384, steps=False), orc.cast_rays(ref, dims, start, d, dist, 384)
     assert np.array_equal(g["hit"], r["hit"])
     ctx.close()
 
@@ -159,6 +157,6 @@ def test_device_upload_at_odd_sizes(gpu, orc, dims):
     d = rng.normal(size=(n, 3)).astype(np.float32)
     d[:, 1] = np.abs(d[:, 1])
     dist = np.full(n, 300, np.int32)
-    g, r = ray_orders.cast_rays(ctx, start, d, dist, 384, steps=False), orc.cast_rays(world, dims, start, d, dist, 384)
+    g, r = ctx.cast_rays(start, d, dist, 384, steps=False), orc.cast_rays(world, dims, start, d, dist, 384)
     assert np.array_equal(g["hit"], r["hit"])
     ctx.close()

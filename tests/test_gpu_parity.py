@@ -7,8 +7,6 @@ the oracle's with the shadow cutoff off, and never above them with it on."""
 import numpy as np
 import pytest
 
-import ray_orders
-
 pytestmark = pytest.mark.gpu
 
 RGB_TOL = 1  # LSB per channel
@@ -165,7 +163,7 @@ def test_cast_rays_match_oracle(gpu, orc):
     dist[:50] = 0
     ctx = gpu.Context(sc.dims)
     ctx.upload(wdf)
-    g = ray_orders.cast_rays(ctx, start, d, dist, 384)
+    g = ctx.cast_rays(start, d, dist, 384)
     r = orc.cast_rays(wdf, sc.dims, start, d, dist, 384)
     for k in ("hit", "face", "steps"):
         bad = np.nonzero(g[k] != r[k])[0]
@@ -417,7 +415,7 @@ def test_cast_rays_entering_from_one_cell_outside(gpu, orc, dims):
     wdf = ctx.download()
     start, d = entering_rays(dims, 1500, rng)
     dist = np.full(start.shape[0], 384, np.int32)
-    g = ray_orders.cast_rays(ctx, start, d, dist, 384)
+    g = ctx.cast_rays(start, d, dist, 384)
     r = orc.cast_rays(wdf, dims, start, d, dist, 384)
     for k in ("hit", "face", "steps"):
         bad = np.nonzero(g[k] != r[k])[0]
@@ -462,7 +460,7 @@ def test_cast_rays_near_and_past_the_grid_faces(gpu, orc):
     d = np.concatenate(dirs).astype(np.float32)
     dist = rng.integers(1, 200, start.shape[0]).astype(np.int32)
     for budget in (384, 1 << 24):
-        g = ray_orders.cast_rays(ctx, start, d, dist if budget == 384 else np.full_like(dist, budget), budget)
+        g = ctx.cast_rays(start, d, dist if budget == 384 else np.full_like(dist, budget), budget)
         r = orc.cast_rays(wdf, dims, start, d, dist if budget == 384 else np.full_like(dist, budget), budget)
         for k in ("hit", "face", "steps"):
             bad = np.nonzero(g[k] != r[k])[0]
@@ -490,7 +488,7 @@ def test_cast_rays_extreme_values_match_oracle(gpu, orc):
     ctx.upload(wdf)
     for budget in (384, 1 << 24):
         dist = np.full(n, budget, np.int32)
-        g = ray_orders.cast_rays(ctx, starts, dirs, dist, budget)
+        g = ctx.cast_rays(starts, dirs, dist, budget)
         r = orc.cast_rays(wdf, sc.dims, starts, dirs, dist, budget)
         for k in ("hit", "face", "steps"):
             assert np.array_equal(g[k], r[k]), (budget, k, g[k], r[k])
@@ -526,7 +524,7 @@ def test_cast_rays_fuzz_small_and_odd_grids(gpu, orc):
         start, d = start.astype(np.float32), d.astype(np.float32)
         dist = rng.integers(0, 300, m).astype(np.int32)
         for steps in (True, False):
-            g = ray_orders.cast_rays(ctx, start, d, dist, 256, steps=steps)
+            g = ctx.cast_rays(start, d, dist, 256, steps=steps)
             r = orc.cast_rays(wdf, dims, start, d, dist, 256)
             keys = ("hit", "face", "steps") if steps else ("hit", "face")
             for k in keys:
@@ -728,8 +726,8 @@ def test_cast_rays_cutoff_without_steps(gpu, orc):
     d = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
     dist = np.full(n, 384, np.int32)
     r = orc.cast_rays(wdf, sc.dims, start, d, dist, 384)
-    full = ray_orders.cast_rays(ctx, start, d, dist, 384)
-    cut = ray_orders.cast_rays(ctx, start, d, dist, 384, steps=False)
+    full = ctx.cast_rays(start, d, dist, 384)
+    cut = ctx.cast_rays(start, d, dist, 384, steps=False)
     for k in ("hit", "face"):
         assert np.array_equal(full[k], r[k]) and np.array_equal(cut[k], r[k]), k
     assert same_floats(cut["hit_pos"], r["hit_pos"]) and np.array_equal(full["steps"], r["steps"])
@@ -748,7 +746,7 @@ def test_pin_rays_match_oracle(gpu, orc):
         dist = np.full(start.shape[0], 384, np.int32)
         ctx = gpu.Context(dims)
         ctx.upload(w)
-        g = ray_orders.cast_rays(ctx, start, d, dist, 384)
+        g = ctx.cast_rays(start, d, dist, 384)
         r = orc.cast_rays(w, dims, start, d, dist, 384)
         for k in ("hit", "face", "steps"):
             assert np.array_equal(g[k], r[k]), "%s: %s gpu %s oracle %s" % (make.__name__, k, g[k], r[k])

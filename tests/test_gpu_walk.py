@@ -1,13 +1,11 @@
 """The written-out walk (vrt_device.h: cast_ray, run_walk) where its arithmetic
 differs in form from the shader's: whole coordinates after a jump, ties, walks
 that leave the grid by a low face or by the x-y edge, starts outside its range,
-directions so long that a jump ends beyond 2^31.
+directions so long that a jump ends beyond 2^31, components near 0.
 Against the oracle's castRay, bit for bit, for 32-bit byte offsets and 32-bit
 indices."""
 import numpy as np
 import pytest
-
-import ray_orders
 
 pytestmark = pytest.mark.gpu
 
@@ -21,7 +19,7 @@ def compare(gpu, orc, world, dims, start, d, dist, budget=256):
     ctx.upload(world)
     r = orc.cast_rays(world, dims, start, d, dist, budget)
     for steps in (True, False):
-        g = ray_orders.cast_rays(ctx, start, d, dist, budget, steps=steps)
+        g = ctx.cast_rays(start, d, dist, budget, steps=steps)
         for k in ("hit", "face", "steps") if steps else ("hit", "face"):
             bad = np.nonzero(g[k] != r[k])[0]
             assert bad.size == 0, "%s differs for %d rays, first start %s dir %s: %s, oracle %s" % (
@@ -119,6 +117,25 @@ def test_long_directions(gpu, orc, dims, axis):
 
 
 @pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
+def test_components_near_zero(gpu, orc, dims):
+    """Components on both sides of 2^-60 and 2^-19, and around the -1e-6 whose
+    step size is infinite; starts near the low faces."""
+    rng = np.random.default_rng(47)
+    world = jumps_and_solids(rng, dims)
+    n = 40000
+    start = np.stack([rng.uniform(2.0 ** -20, min(s, 48), n) for s in dims], 1)
+    low = rng.random((n, 3)) < 0.1
+    start[low] = 2.0 ** rng.uniform(-20, 0, int(low.sum()))
+    d = rng.normal(size=(n, 3))
+    small = rng.random((n, 3)) < 0.3
+    d[small] = rng.choice([-1.0, 1.0], int(small.sum())) * 2.0 ** rng.uniform(-62, -12, int(small.sum()))
+    step = rng.random((n, 3)) < 0.05
+    d[step] = np.float32(-1e-6) * (1 + rng.integers(-4, 5, int(step.sum())) * 2.0 ** -23)
+    r = compare(gpu, orc, world, dims, start, d, rng.integers(1, 200, n))
+    assert int((r["hit"] >= 0).sum()) > 1000
+
+
+@pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
 def test_longest_jumps_that_run_walk_takes(gpu, orc, dims):
     """Components up to 2^6, jumps and budgets up to 2^24: positions up to 2^30,
     short of where a cell saturates."""
@@ -143,3 +160,39 @@ def test_step_count_of_a_jump_beyond_two_to_the_31(gpu, orc):
     world[5 + dims[0] * (6 + dims[1] * 5)] = np.float32(-2.0).view(np.int32)
     r = compare(gpu, orc, world, dims, [[5.5, 5.5, 5.5]], [[0.3, 2.0 ** 32, 0.3]], [200], 200)
     assert r["steps"].tolist() == [2]
+
+
+@pytest.mark.parametrize("dims", GRIDS, ids=["byte_offset32", "index32"])
+@pytest.mark.parametrize("axis", [0, 1, 2], ids="xyz")
+def test_primary_rays_with_a_component_near_zero(gpu, orc, dims, axis):
+    """Frames whose rays all have one small component, down to below 2^-60, by a
+    scaled rotation; or one near the -1e-6 whose step size is infinite."""
+    rng = np.random.default_rng(48 + axis)
+    world = jumps_and_solids(rng, dims)
+    ctx = gpu.Context(dims)
+    ctx.upload(world)
+    size = (72, 56)
+    t = gpu.Target(*size, depth=True, aux=True)
+    hits = 0
+    for scale in [2.0 ** -k for k in (10, 19, 21, 35, 50, 58, 62)] + [-1e-6]:
+        f = gpu.frame_defaults(dims[0], *size)
+        f.cam_pos[:] = [0.4 * dims[0], 0.5 * dims[1], 0.3 * dims[2]]
+        m = np.asarray(gpu.camera_matrix(0.3, 0.7), np.float32).reshape(4, 4)  # columns
+        m[:3, axis] *= np.float32(scale)
+        if scale < 0:  # -1e-6 times the depth component of the pixel
+            m[:3, axis] = 0.0
+            m[2, axis] = np.float32(scale)
+        f.rotate_matrix[:] = m.ravel().tolist()
+        f.aspect_ratio = size[0] / size[1]
+        for depth_view in (0, 1):
+            f.view_depth_field = depth_view
+            ctx.draw(t, frame=f)
+            g, r = t.download(), orc.render(world, dims, f, *size)
+            for k in ("hit", "face", "steps", "shadow_eval", "shadow_occ"):
+                bad = np.argwhere(g[k] != r[k])
+                assert bad.size == 0, (scale, depth_view, k, len(bad), bad[0].tolist())
+            same = (g["depth"].view(np.uint32) == r["depth"].view(np.uint32)) | (np.isnan(g["depth"]) & np.isnan(r["depth"]))
+            assert same.all(), (scale, depth_view)
+        hits += int((r["hit"] >= 0).sum())
+    assert hits > 500
+    ctx.close()

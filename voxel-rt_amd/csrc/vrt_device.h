@@ -398,7 +398,8 @@ __device__ __forceinline__ void walk_generic(const GridDesc& g, float sx, float 
 // takes up the 1.
 //
 // Which rays: those whose direction components lie in [2^-19, 2^6] in
-// magnitude and whose start coordinates lie in [2^-20, 2^22] (start_walk).  On an
+// magnitude (kWide: from 2^-60, with 1e-6 added too) and whose start coordinates
+// lie in [2^-20, 2^22] (start_walk).  On an
 // ascending axis s then stays at least 2^-20, where the hardware's fraction is
 // the rounded difference; on a descending one s may fall below 0 only on its
 // way out of the grid (below).  Only the low end of a cell is clamped (lo:
@@ -650,11 +651,20 @@ __device__ __forceinline__ void run_walk(Idx32, const int32_t* vox, float lim, u
 // The walk's state at a ray's start (arguments as cast_ray's), for rays that
 // run_walk takes; false for any other.
 //
+// kWide (a frame's primary rays where the lanes count): a lane that goes to
+// walk_generic makes its wave walk twice, one form after the other.  Along the
+// horizon a component passes through 0 and a pixel in 700 lies below 2^-19: few,
+// but in a frame's longest waves, which end it where it has few tiles or its
+// rays run far.  Depth view, 1920x1080 in a 512x512x3700 grid: 399 us, from 2^-19
+// 503; 960x540 261 and 374; 800x600 in a small world 2 to 3% less.  (Sending the
+// whole wave to walk_generic instead: 402, 265 and 1% more everywhere.  Other rays
+// do not gain: 16 views in one launch 1% slower, lists of few rays 3%.)
+//
 // The first cell and intersects.  From a hit: as after a jump, for a start
 // inside the grid (any other takes walk_generic).  Else: the reference's
 // formulas.  (The camera's distances to its cell's boundaries made with the
 // frame instead of by every lane: no gain, small frames 2% slower.)
-template <typename IX, bool kHit>
+template <typename IX, bool kHit, bool kWide>
 __device__ __forceinline__ bool start_walk(const GridDesc& g, float px, float py, float pz, float dx, float dy,
                                            float dz, Walk& w) {
     const float sx = kHit ? px + dx * 0.001f : px, sy = kHit ? py + dy * 0.001f : py,
@@ -663,11 +673,13 @@ __device__ __forceinline__ bool start_walk(const GridDesc& g, float px, float py
     w.sx = mx ? -sx : sx;
     w.sy = my ? -sy : sy;
     w.sz = mz ? -sz : sz;
-    // |d| >= 2^-19 keeps |d + 1e-6| in range too.  min and max pass over a
-    // NaN; the comparisons of s (NaN where d is) or the sum do not.
-    const float lo = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
+    // |d| >= 2^-19 keeps |d + 1e-6| in range too; kWide tests both.  min and max
+    // pass over a NaN; the comparisons of s (NaN where d is) or the sum do not.
+    const float bx = fabsf(dx + 0.000001f), by = fabsf(dy + 0.000001f), bz = fabsf(dz + 0.000001f);
+    float lo = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
+    if constexpr (kWide) lo = fminf(lo, fminf(fminf(bx, by), bz));
     const float hi = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz));
-    bool fast = (lo >= 0x1p-19f) & (hi <= 0x1p6f);
+    bool fast = (lo >= (kWide ? 0x1p-60f : 0x1p-19f)) & (hi <= 0x1p6f);
     if constexpr (kHit) {
         w.ix = __builtin_amdgcn_fractf(w.sx);
         w.iy = __builtin_amdgcn_fractf(w.sy);
@@ -678,9 +690,9 @@ __device__ __forceinline__ bool start_walk(const GridDesc& g, float px, float py
         fast &= (fminf(fminf(sx, sy), sz) >= 0x1p-20f) & (fmaxf(fmaxf(sx, sy), sz) <= 0x1p22f) & (sum == sum);
     }
     if (!fast) return false;
-    w.ddx = rcp_fast(fabsf(dx + 0.000001f));
-    w.ddy = rcp_fast(fabsf(dy + 0.000001f));
-    w.ddz = rcp_fast(fabsf(dz + 0.000001f));
+    w.ddx = rcp_fast(bx);
+    w.ddy = rcp_fast(by);
+    w.ddz = rcp_fast(bz);
     w.rx = rcp_fast(fabsf(dx));
     w.ry = rcp_fast(fabsf(dy));
     w.rz = rcp_fast(fabsf(dz));
@@ -739,24 +751,14 @@ __device__ __forceinline__ bool start_walk(const GridDesc& g, float px, float py
 //
 // kLanes: h.iters is the ray's own iterations (a step map or the depth view
 // shows them); else the lanes' h.iters only add up to the wave's.
-template <typename IX, bool kHit, bool kLanes>
+template <typename IX, bool kHit, bool kLanes, bool kWide = false>
 __device__ __forceinline__ void cast_ray(const GridDesc& g, float px, float py, float pz, float dx, float dy,
                                          float dz, float lim, Hit& h, int32_t ytop) {
     bool general = true, again = false;
     h.iters = 0;
     if constexpr (!std::is_same_v<IX, Idx64>) {
         Walk w;
-        // One lane that run_walk does not take sends the wave to walk_generic
-        // where the lanes count (a depth view or step map, whose walks are
-        // long): two walks one after the other cost the wave the time of both.
-        // Such lanes are few (a pixel in 700 along the horizon, where a component
-        // is below 2^-19), but their waves are a frame's longest.  Depth view,
-        // 1920x1080 in a 512x512x3700 grid: 400 us, each lane by its own walk
-        // 511.  (In shaded frames no gain, and at 3840x2160 1% more for the test.
-        // Taking such rays too, by a test of |d + 1e-6|: the same for the depth
-        // view, 16 views in one launch 1% slower.)
-        const bool fast = start_walk<IX, kHit>(g, px, py, pz, dx, dy, dz, w);
-        if (kLanes ? __ballot(!fast) == 0 : fast) {
+        if (start_walk<IX, kHit, kWide>(g, px, py, pz, dx, dy, dz, w)) {
             w.tb = dy > 0.0f ? -1.0f - (float)ytop : -__builtin_inff();
             run_walk<kLanes>(IX{}, g.vox, lim, __ballot(0.0f < lim), w);
             auto flip = [](int32_t nst, float v) { return nst < 0 ? -v : v; };
@@ -812,7 +814,7 @@ __device__ __forceinline__ void shade_pixel(const GridDesc& g, const FrameDesc& 
     // output of this draw (no depth view, no step map): a ray that stops
     // there misses, as the reference's walk would.
     Hit h;
-    cast_ray<IX, false, kLanes>(g, f.cam_pos[0], f.cam_pos[1], f.cam_pos[2], d0, d1, d2, F.render_lim, h,
+    cast_ray<IX, false, kLanes, kLanes>(g, f.cam_pos[0], f.cam_pos[1], f.cam_pos[2], d0, d1, d2, F.render_lim, h,
                         F.primary_cutoff != 0 ? top : INT32_MAX);
     iters = h.iters;
     uint32_t eval = 0, occ = 0;
